@@ -255,7 +255,9 @@ int simpler_render_host(simpler_scene *scene, int64_t n_photons,
  * for callers that cannot allocate device memory: tight serving loops,
  * harnesses that forbid hipMalloc).  The array holds a 256 B header plus at
  * most 8,388,608 image floats (32 MiB, a 256 x 256 x 128 image); larger
- * images fail with SIMPLER_ERR_INVALID.  Each device the library runs on
+ * images fail with SIMPLER_ERR_INVALID.  What the image leaves of the array
+ * serves as the launch's next-event stacks (a launch without them gives the
+ * same image and counts; few photons then take up to eight times longer).  Each device the library runs on
  * holds one copy until the process ends, and every call on that device
  * shares it (the last call's contents stay): calls that overlap on one
  * device -- on two streams or two contexts at once -- race and must be

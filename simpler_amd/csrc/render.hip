@@ -7,7 +7,8 @@
 // reference renderer/src/photon.cpp:19-136,266-340, scene.cpp:385-946):
 //
 //   loop:
-//     fetch   lanes without a photon take the next photon indices with one
+//     fetch   lanes without work take next-event sub-paths from their wave's
+//             stack (render kernels), else the next photon indices with one
 //             atomic per wave (wave-aggregated work queue), so lanes regenerate
 //             independently and no lane waits for the slowest photon;
 //     events  lanes whose march segment ended run the face / sensor / scatter /
@@ -36,7 +37,8 @@
 
 namespace simpler {
 
-enum { PH_DIRECT = 0, PH_NEE = 1, PH_FLIGHT = 2 };
+// PH_JOB: a next-event sub-path that a lane took from its wave's stack
+enum { PH_DIRECT = 0, PH_NEE = 1, PH_FLIGHT = 2, PH_JOB = 3 };
 enum { ST_MARCH = 0, ST_SEG_END = 1, ST_NEED = 2, ST_INIT = 3, ST_DONE = 4, ST_RMARCH = 5, ST_REND = 6, ST_MREV = 7 };
 // kernel modes: image render, per-ray record, adjoint of an image objective
 // (backward runs inline), adjoint of a per-ray objective, per-ray record with
@@ -59,6 +61,7 @@ constexpr int kBlock = 256;
 constexpr int kJtabLds = 128;  // Bessel table intervals staged in LDS (8 KiB)
 constexpr int kJtabLdsBatch = 1024;  // float4 (16 KiB): a batch's per-order tables in LDS
 constexpr int kMaxMode = 7;          // highest Bessel order (check_desc)
+constexpr int kJobVec = 4;           // float4 per entry of a next-event stack
 
 struct RenderArgs {
     float *image;
@@ -107,6 +110,12 @@ struct RenderArgs {
     // fields), for
     // nee_skip; null: every next-event sub-path is traced
     const int *nee_cut;
+    // next-event stacks of the render kernels (see nee_push): nq_cap entries
+    // of kJobVec float4 for each of the first nq_waves waves of the grid;
+    // wave_photons: photons a wave traces at a time (64 unless the launch has
+    // fewer photons than lanes)
+    float4 *nq;
+    int nq_cap, nq_waves, wave_photons;
     // forward renders of spline fields (nee_cut null): nee_fwd != 0 skips
     // the next-event sub-paths that cannot reach the image, with
     // nee_g >= |grad n| >= |grad n| / n over the block
@@ -196,6 +205,12 @@ struct Lane {
     // adjoint state keeps the compiler from holding that state in registers
     // (it stays in scratch memory).
     bool adj = false;
+    // the wave's next-event stack (render kernels): base, capacity and the
+    // number of entries held (LDS)
+    float4 *q = nullptr;
+    uint32_t qcap = 0;
+    volatile uint32_t *qn = nullptr;
+    int cfg = 0;  // batched renders: the photon's configuration
 };
 
 __device__ __forceinline__ void count(Lane &L, int k) { atomicAdd(L.cnt + k, 1u); }
@@ -834,11 +849,103 @@ __device__ __forceinline__ bool nee_skip(const Lane &L, f3 d) {
     return false;
 }
 
+// The next-event stack.  A photon's next-event sub-paths depend on the main
+// path only through the state at their vertex, and each draws from a random
+// sub-stream of its own, so the lane that walks the main path leaves them on a
+// stack of its wave (global memory, L2 resident; no other wave touches it)
+// and walks on; a lane without work takes the newest entry before it takes a
+// new photon.  A photon is then a chain of at most one main path and one
+// sub-path -- about 3e4 steps for a 100 mm time gate at 5 um -- instead of
+// the main path with every sub-path in turn (up to 7e5), and that chain is
+// what a launch waits for when its photons run out.  With a full stack the
+// lane traces the sub-path itself and then resumes its main path.  Measured
+// (one lane per photon -> stacks): 5,000 photons of the 10 um Bessel scene
+// 51 -> 10 ms, 2^22 of the 5 um scene 554 -> 478 ms, a sweep of 256
+// configurations and 1.04e6 photons 1448 -> 406 ms, 2^17 of the 64^3 spline
+// 529 -> 172 ms, 2^15 of 16 point sources 1.75 -> 0.22 s.
+//
+// nee_push: called by the lanes at a vertex (any subset of the wave); false
+// when the stack is full.
+template <int FIELD>
+__device__ __forceinline__ bool nee_push(Lane &L) {
+    const unsigned long long m = __ballot(1);
+    const int lane = __lane_id(), leader = __ffsll((long long)m) - 1;
+    const uint32_t held = *L.qn;
+    const uint32_t i = held + (uint32_t)__popcll(m & ((1ull << lane) - 1ull));
+    if (lane == leader) *L.qn = min(held + (uint32_t)__popcll(m), L.qcap);
+    if (i >= L.qcap) return false;
+    const Hot &h = L.h;
+    const Cold &c = L.c;
+    float4 *r = L.q + (size_t)i * kJobVec;
+    r[0] = make_float4(h.p.x, h.p.y, h.p.z, h.L);
+    r[1] = make_float4(h.v.x, h.v.y, h.v.z, h.n0);
+    r[2] = make_float4(h.g0.x, h.g0.y, h.g0.z, FIELD == kSources ? h.tau : h.scaling);
+    r[3] = make_float4(__uint_as_float(c.pid_lo), __uint_as_float(c.pid_hi), __int_as_float(c.depth),
+                       __int_as_float(L.cfg));
+    // the wave's vector memory accesses are performed in order; this keeps
+    // the compiler from moving the stores past a later entry's loads
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    return true;
+}
+
+// The direction of the next-event sub-path at the lane's vertex: the first
+// draws of its own sub-stream, which the lane is left on (scene.cpp:20-39 +
+// warp.cpp:22-34: uniform hemisphere about -x).
+__device__ __forceinline__ f3 nee_dir(Lane &L) {
+    Cold &c = L.c;
+    c.stream = 1u + (uint32_t)c.depth;
+    c.draw = 0;
+    float u[2];
+    draw_k<2>(L, u);
+    const float z = u[0], s1 = u[1];
+    const float tmp = sqrtf(1.f - z * z);
+    float sa, ca;
+    sincosf(2.0f * kPi * s1, &sa, &ca);
+    return mk3(-z, ca * tmp, sa * tmp);
+}
+
+__device__ __forceinline__ void nee_begin(Lane &L, f3 d, int phase) {
+    L.h.v = L.h.n0 * d;
+    L.c.phase = phase;
+    L.c.acc = 0.f;
+    L.c.large = kLargeDist;
+    L.c.faces = 0;
+}
+
+// Entry i of the wave's stack as the lane's sub-path.
+template <int FIELD, bool BATCH>
+__device__ __forceinline__ void nee_pop(Lane &L, uint32_t i) {
+    Hot &h = L.h;
+    Cold &c = L.c;
+    const float4 *r = L.q + (size_t)i * kJobVec;
+    const float4 r0 = r[0], r1 = r[1], r2 = r[2], r3 = r[3];
+    h.p = mk3(r0.x, r0.y, r0.z);
+    h.pl = mk3(0.f, 0.f, 0.f);
+    h.L = r0.w;
+    h.Ll = 0.f;
+    c.mv = mk3(r1.x, r1.y, r1.z);
+    h.n0 = r1.w;
+    h.g0 = mk3(r2.x, r2.y, r2.z);
+    if (FIELD == kSources)
+        h.tau = r2.w;
+    else
+        h.scaling = r2.w;
+    c.pid_lo = __float_as_uint(r3.x);
+    c.pid_hi = __float_as_uint(r3.y);
+    c.depth = __float_as_int(r3.z);
+    if (BATCH) {
+        L.cfg = __float_as_int(r3.w);
+        L.v = const_cast<Var *>(L.A.cfgs) + L.cfg;
+    }
+    nee_begin(L, nee_dir(L), PH_JOB);
+    start_segment(L, kLargeDist);
+}
+
 // photon.cpp:111-116 loop head + scene.cpp:866-893 (NEE start).  Forward
 // renders take nee_skip in the spline kernels only: inlined into the Bessel
 // kernel's event code it slows that kernel's march loop by a fifth per step,
 // more than the 11 % of its steps it removes.
-template <int FIELD>
+template <int FIELD, int MODE>
 __device__ __forceinline__ void vertex(Lane &L) {
     const DevScene &S = L.S;
     Hot &h = L.h;
@@ -848,33 +955,33 @@ __device__ __forceinline__ void vertex(Lane &L) {
         return;
     }
     if (S.use_nee && !((double)(h.p.x - S.cam_o.x) < 1e-4)) {
-        c.mp = h.p;
-        c.mv = h.v;
-        c.mL = h.L;
-        if (L.mc) *L.mc = make_float4(h.n0, h.g0.x, h.g0.y, h.g0.z);
         c.main_draw = c.draw;
-        c.stream = 1u + (uint32_t)c.depth;
-        c.draw = 0;
-        // scene.cpp:20-39 + warp.cpp:22-34: uniform hemisphere about -x
-        float u[2];
-        draw_k<2>(L, u);
-        const float z = u[0], s1 = u[1];
-        const float tmp = sqrtf(1.f - z * z);
-        float sa, ca;
-        sincosf(2.0f * kPi * s1, &sa, &ca);
-        h.v = h.n0 * mk3(-z, ca * tmp, sa * tmp);
-        c.phase = PH_NEE;
-        c.acc = 0.f;
-        c.large = kLargeDist;
-        c.faces = 0;
-        if ((L.adj || (FIELD == kSpline && L.A.nee_fwd)) && nee_skip(L, mk3(-z, ca * tmp, sa * tmp))) {  // no splat
-            h.dead = true;
-            h.state = ST_SEG_END;
+        bool walk_on = false;  // no sub-path to trace here
+        if constexpr (MODE == M_RENDER) {
+            if (FIELD == kSpline && L.A.nee_fwd) {
+                const f3 d = nee_dir(L);
+                walk_on = nee_skip(L, d);  // no splat
+                c.stream = 0;
+                c.draw = c.main_draw;
+            }
+            walk_on = walk_on || nee_push<FIELD>(L);
+        }
+        if (!walk_on) {
+            c.mp = h.p;
+            c.mv = h.v;
+            c.mL = h.L;
+            if (L.mc) *L.mc = make_float4(h.n0, h.g0.x, h.g0.y, h.g0.z);
+            const f3 d = nee_dir(L);
+            nee_begin(L, d, PH_NEE);
+            if (L.adj && nee_skip(L, d)) {  // no splat
+                h.dead = true;
+                h.state = ST_SEG_END;
+                return;
+            }
+            if (L.adj) adj_sub_begin(*L.a);
+            start_segment(L, kLargeDist);
             return;
         }
-        if (L.adj) adj_sub_begin(*L.a);
-        start_segment(L, kLargeDist);
-        return;
     }
     scatter_once(L);
 }
@@ -973,7 +1080,10 @@ __device__ __forceinline__ void nee_done(Lane &L, int res) {
             }
         }
     }
-    nee_continue<FIELD>(L);
+    if (MODE == M_RENDER && c.phase == PH_JOB)
+        h.state = ST_NEED;
+    else
+        nee_continue<FIELD>(L);
 }
 
 // End of a march segment: the face / sensor logic of movePhoton
@@ -1013,7 +1123,7 @@ __device__ __forceinline__ void seg_end(Lane &L) {
             ++c.depth;
         }
         if constexpr (adj_image(MODE)) adj_log_main(L, K_DIST, mk3(0.f, 0.f, 0.f));
-        vertex<FIELD>(L);
+        vertex<FIELD, MODE>(L);
         return;
     }
     int res;
@@ -1180,7 +1290,7 @@ namespace simpler {
 // reference's axis = x form).
 // SPLAT: 0 = every lane issues its splat's atomics, 1 = wave-aggregated
 // splats (wave_splat after the event phase); an autotuner candidate.
-static_assert(5 * (sizeof(Cold) * kBlock + sizeof(uint32_t) * C_N + sizeof(float4) * (4 * kJtabLds + kBlock)) <=
+static_assert(5 * (sizeof(Cold) * kBlock + sizeof(uint32_t) * (C_N + kBlock / 64) + sizeof(float4) * (4 * kJtabLds + kBlock)) <=
                   160 * 1024,
               "five single-scene Bessel workgroups must fit one CU's LDS");
 
@@ -1191,7 +1301,10 @@ k_render(DevScene S, RenderArgs A) {
     __shared__ uint32_t cnt[C_N];
     __shared__ float4 jlds[JLDS ? (BATCH ? kJtabLdsBatch : 4 * kJtabLds) : 1];
     __shared__ float4 mcache[kBlock];
+    __shared__ uint32_t nheld[kBlock / 64];  // entries of each wave's next-event stack
+    constexpr bool STACK = MODE == M_RENDER;
     if (threadIdx.x < C_N) cnt[threadIdx.x] = 0u;
+    if (STACK && (threadIdx.x & 63) == 0) nheld[threadIdx.x >> 6] = 0u;
     if (JLDS) {
         const float4 *src = BATCH ? A.jtab_base : S.jtab;
         const int nj = BATCH ? A.jtab_len : 4 * S.jtab_n;
@@ -1215,16 +1328,45 @@ k_render(DevScene S, RenderArgs A) {
     Lane L{h, cold[threadIdx.x], vp, S, A, cnt, nullptr, &mcache[threadIdx.x], SPLAT ? &ps : nullptr,
            MODE == M_JVP ? &tan : nullptr};
     const int lane = __lane_id();
+    if (STACK) {
+        const int wave = (int)((blockIdx.x * blockDim.x + threadIdx.x) >> 6);
+        L.qn = &nheld[threadIdx.x >> 6];
+        L.qcap = __builtin_amdgcn_readfirstlane(wave < A.nq_waves ? A.nq_cap : 0);
+        L.q = A.nq + (size_t)__builtin_amdgcn_readfirstlane(wave) * A.nq_cap * kJobVec;
+    }
+    bool left = true;  // photons left in the launch's queue (uniform)
     unsigned long long wave_steps = 0;  // ER steps of the wave (uniform)
     while (true) {
-        // fetch: one atomic per wave for all lanes that need a photon
-        const unsigned long long need = __ballot(h.state == ST_NEED);
-        if (need) {
+        // fetch: first the wave's next-event stack, then new photons, one
+        // atomic per wave for all lanes that take one
+        unsigned long long need = __ballot(h.state == ST_NEED);
+        if (STACK && need) {
+            const uint32_t held = __builtin_amdgcn_readfirstlane(*L.qn);
+            if (held) {
+                const uint32_t want = (uint32_t)__popcll(need);
+                const uint32_t rank = (uint32_t)__popcll(need & ((1ull << lane) - 1ull));
+                if (lane == 0) *L.qn = held - min(held, want);
+                __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+                if (h.state == ST_NEED && rank < held) {
+                    nee_pop<FIELD, BATCH>(L, held - 1u - rank);
+                }
+                // lanes that found no entry take a photon
+                need = __ballot(h.state == ST_NEED && rank >= held);
+            }
+        }
+        if (STACK && need && left && A.wave_photons < 64) {  // fewer photons than lanes: spread over the waves
+            const int mains = __popcll(__ballot(h.state != ST_NEED && L.c.phase != PH_JOB));
+            const int room = max(A.wave_photons - mains, 0);
+            while (__popcll(need) > room) need &= need - 1ull;
+        }
+        if (need && left) {
             const int leader = __ffsll((long long)need) - 1;
             unsigned long long base = 0;
             if (lane == leader) base = atomicAdd(A.work, (unsigned long long)__popcll(need));
-            base = __shfl(base, leader);
-            if (h.state == ST_NEED) {
+            base = (unsigned long long)(uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)base, leader) |
+                   (unsigned long long)(uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(base >> 32), leader) << 32;
+            left = base + __popcll(need) < A.n;
+            if ((need >> lane) & 1ull) {
                 const unsigned long long rank = __popcll(need & ((1ull << lane) - 1ull));
                 const unsigned long long idx = base + rank;
                 if (idx < A.n) {
@@ -1243,20 +1385,21 @@ k_render(DevScene S, RenderArgs A) {
                         }
                         pid = gi - A.prefix[lo];
                         L.v = const_cast<Var *>(A.cfgs + lo);  // its image pointer is set per launch
+                        L.cfg = lo;
                     }
                     L.c.pid_lo = (uint32_t)pid;
                     L.c.pid_hi = (uint32_t)(pid >> 32);
                     h.state = ST_INIT;
-                } else {
-                    h.state = ST_DONE;
                 }
             }
         }
         if (h.state == ST_INIT) photon_init<FIELD, MODE>(L);
         if (h.state == ST_SEG_END) seg_end<FIELD, MODE>(L);
         if (SPLAT) wave_splat(ps, A);
-        if (__ballot(h.state != ST_DONE) == 0ull) break;
-        if (__ballot(h.state == ST_MARCH) == 0ull) continue;
+        if (__ballot(h.state == ST_MARCH) == 0ull) {
+            if (__ballot(h.state != ST_NEED) == 0ull && !left && (!STACK || *L.qn == 0u)) break;
+            continue;
+        }
         FieldP F = L.v->f;
         if (BATCH && JLDS) F.jtab = jlds + (F.jtab - A.jtab_base);
         float Lcut = L.v->Lcut;
@@ -1550,6 +1693,8 @@ struct simpler_ctx {
     hipStream_t own = nullptr;
     hipStream_t cur = nullptr;
     unsigned long long *d_scratch = nullptr;  // [0..7] work, [8..15] counters
+    float4 *d_nq = nullptr;  // next-event stacks of the first nq_waves waves of a render grid
+    int nq_waves = 0;
     int num_cu = 256;
     int block = 256, spc = 32, bpc = 4;
     int splat = 0;  // splat strategy: 0 per-lane atomics, 1 wave-aggregated
@@ -1860,9 +2005,24 @@ static int bessel_variant(const DevScene &S) {
     return 3 * S.mode + (axis_zframe(S) ? 2 : (S.general_axis ? 1 : 0));
 }
 
+// Next-event stacks: 64 entries for each wave of five workgroups of 256 per
+// CU, the largest render grid that is resident (waves of larger grids, and
+// the entries past a full stack, trace inline).
+constexpr int kStackEntries = 64, kStackWavesPerCU = 5 * kBlock / 64;
+
+// The launch's grid and the photons each wave traces at a time: a launch with
+// fewer photons than lanes spreads them over its waves, whose other lanes
+// take the next-event sub-paths.
+static void render_shape(const simpler_ctx *ctx, RenderArgs &A, int &blocks) {
+    blocks = std::max(1, ctx->num_cu * ctx->bpc);
+    const uint64_t waves = (uint64_t)blocks * (uint64_t)(ctx->block / 64);
+    A.wave_photons = (int)std::max<uint64_t>(1, std::min<uint64_t>(64, (A.n + waves - 1) / waves));
+}
+
 template <int MODE>
-static void launch_render(simpler_ctx *ctx, int field, const DevScene &S, const RenderArgs &A) {
-    const int blocks = std::max(1, ctx->num_cu * ctx->bpc);
+static void launch_render(simpler_ctx *ctx, int field, const DevScene &S, RenderArgs A) {
+    int blocks = 0;
+    render_shape(ctx, A, blocks);
     const dim3 grid(blocks), block(ctx->block);
     switch (field) {
         case SIMPLER_FIELD_BESSEL:
@@ -1972,7 +2132,10 @@ int simpler_ctx_create(int device, simpler_ctx **out) {
     scratch_init(device);
     if (hipStreamCreateWithFlags(&ctx->own, hipStreamNonBlocking) != hipSuccess ||
         hipEventCreateWithFlags(&ctx->handoff, hipEventDisableTiming) != hipSuccess ||
-        hipMalloc(&ctx->d_scratch, 16 * sizeof(unsigned long long)) != hipSuccess) {
+        hipMalloc(&ctx->d_scratch, 16 * sizeof(unsigned long long)) != hipSuccess ||
+        hipMalloc(&ctx->d_nq, (size_t)(ctx->nq_waves = ctx->num_cu * kStackWavesPerCU) * kStackEntries * kJobVec *
+                                  sizeof(float4)) != hipSuccess) {
+        (void)hipFree(ctx->d_scratch);
         if (ctx->handoff) (void)hipEventDestroy(ctx->handoff);
         if (ctx->own) (void)hipStreamDestroy(ctx->own);
         delete ctx;
@@ -1989,6 +2152,7 @@ int simpler_ctx_destroy(simpler_ctx *ctx) {
     (void)hipSetDevice(ctx->device);
     (void)hipStreamSynchronize(ctx->cur);
     (void)hipFree(ctx->d_scratch);
+    (void)hipFree(ctx->d_nq);
     (void)hipFree(ctx->d_log);
     (void)hipFree(ctx->d_adj);
     (void)hipFree(ctx->d_jobs);
@@ -2053,7 +2217,8 @@ int simpler_ctx_set_tuning(simpler_ctx *ctx, int block_size, int steps_per_chunk
 
 static int render_impl(simpler_scene *sc, int64_t n_photons, int64_t n_total, uint64_t seed, uint64_t offset,
                        float *image, int X, int Y, int Z, int accumulate, bool record, float *rp, float *rd, float *rL,
-                       int32_t *rs, unsigned long long *words = nullptr);
+                       int32_t *rs, unsigned long long *words = nullptr, float4 *stacks = nullptr,
+                       size_t stack_vec = 0);
 
 int simpler_autotune(simpler_scene *sc, int64_t n_photons, int X, int Y, int Z, int *block_out, int *spc_out,
                      int *bpc_out, float *ms_out) {
@@ -2573,13 +2738,18 @@ static void nee_forward(const simpler_ctx *ctx, const simpler_scene *sc, const D
     }
 }
 
-// words: the launch's work queue ([0]) and counters ([8..15]); the
-// context's buffer unless the caller brings its own.
+// words: the launch's work queue ([0]) and counters ([8..15]), with stacks
+// its next-event stacks (stack_vec float4); the context's buffers unless the
+// caller brings its own.
 static int render_impl(simpler_scene *sc, int64_t n_photons, int64_t n_total, uint64_t seed, uint64_t offset,
                        float *image, int X, int Y, int Z, int accumulate, bool record, float *rp, float *rd, float *rL,
-                       int32_t *rs, unsigned long long *words) {
+                       int32_t *rs, unsigned long long *words, float4 *stacks, size_t stack_vec) {
     simpler_ctx *ctx = sc->ctx;
-    if (!words) words = ctx->d_scratch;
+    if (!words) {
+        words = ctx->d_scratch;
+        stacks = ctx->d_nq;
+        stack_vec = (size_t)ctx->nq_waves * kStackEntries * kJobVec;
+    }
     int rc = scene_ready(sc);
     if (rc) return rc;
     if (n_photons < 0) return fail(ctx, SIMPLER_ERR_INVALID, "n_photons must be >= 0");
@@ -2609,6 +2779,9 @@ static int render_impl(simpler_scene *sc, int64_t n_photons, int64_t n_total, ui
     A.rec_L = rL;
     A.rec_s = rs;
     A.spc = ctx->spc;
+    A.nq = stacks;
+    A.nq_waves = ctx->nq_waves;
+    A.nq_cap = (int)std::min<size_t>(kStackEntries, stack_vec / ((size_t)ctx->nq_waves * kJobVec));
     // zero work queue + counters (a fill kernel: safe under graph capture)
     hipLaunchKernelGGL(k_fill_u64, dim3(1), dim3(64), 0, ctx->cur, words, 16);
     if (!record && !accumulate) {
@@ -2697,8 +2870,11 @@ int simpler_render_host_noalloc(simpler_scene *sc, int64_t n_photons, int64_t n_
     const size_t bytes = (size_t)X * Y * Z * sizeof(float);
     HIP_TRY(ctx, hipSetDevice(ctx->device));
     if (accumulate) HIP_TRY(ctx, hipMemcpyAsync(img, image_host, bytes, hipMemcpyHostToDevice, ctx->cur));
+    // the next-event stacks take what the image leaves of the array
+    const size_t pix4 = (bytes + sizeof(float4) - 1) / sizeof(float4);
     const int rc = render_impl(sc, n_photons, n_total, seed, offset, img, X, Y, Z, accumulate, false, nullptr,
-                               nullptr, nullptr, nullptr, words);
+                               nullptr, nullptr, nullptr, words, reinterpret_cast<float4 *>(img) + pix4,
+                               kNoAllocPixels / 4 - pix4);
     if (rc) return rc;
     HIP_TRY(ctx, hipMemcpyAsync(image_host, img, bytes, hipMemcpyDeviceToHost, ctx->cur));
     if (stats) return read_counters(ctx, words, stats);
@@ -3237,6 +3413,9 @@ static int batch_launch(simpler_batch *b, float *images, int accumulate, hipStre
     A.n_cfg = b->n_cfg;
     A.jtab_base = b->d_jtab;
     A.jtab_len = b->jtab_len;
+    A.nq = ctx->d_nq;
+    A.nq_waves = ctx->nq_waves;
+    A.nq_cap = kStackEntries;
     hipLaunchKernelGGL(k_fill_u64, dim3(1), dim3(64), 0, stream, ctx->d_scratch, 16);
     hipLaunchKernelGGL(k_cfg_images, dim3((b->n_cfg + 255) / 256), dim3(256), 0, stream, b->d_cfgs, b->n_cfg,
                        b->d_img, images, (size_t)b->X * b->Y * b->Z);
@@ -3246,7 +3425,8 @@ static int batch_launch(simpler_batch *b, float *images, int accumulate, hipStre
         hipLaunchKernelGGL(k_fill_f32, dim3(blocks), dim3(256), 0, stream, images, npix, 0.0f);
     }
     if (b->total > 0) {
-        const int blocks = std::max(1, ctx->num_cu * ctx->bpc);
+        int blocks = 0;
+        render_shape(ctx, A, blocks);
         if (b->field == SIMPLER_FIELD_SOURCES)
             hipLaunchKernelGGL((k_render<kSources, M_RENDER, true>), dim3(blocks), dim3(ctx->block), 0, stream, b->S,
                                A);
@@ -3257,6 +3437,7 @@ static int batch_launch(simpler_batch *b, float *images, int accumulate, hipStre
                 if (k) hipLaunchKernelGGL(k_fill_u64, dim3(1), dim3(64), 0, stream, ctx->d_scratch, 1);
                 A.offset = b->g_start[k];
                 A.n = b->g_count[k];
+                render_shape(ctx, A, blocks);
                 const dim3 grid(blocks), block(ctx->block);
                 switch (b->g_mode[k]) {
                     case 0: batch_bessel_launch<0>(grid, block, stream, b->S, A); break;
