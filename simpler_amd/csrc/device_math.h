@@ -19,7 +19,16 @@ __device__ __forceinline__ f3 operator-(f3 a, f3 b) { return f3{a.x - b.x, a.y -
 __device__ __forceinline__ f3 operator*(float s, f3 a) { return f3{s * a.x, s * a.y, s * a.z}; }
 __device__ __forceinline__ f3 operator*(f3 a, float s) { return f3{s * a.x, s * a.y, s * a.z}; }
 __device__ __forceinline__ f3 operator/(f3 a, float s) { return f3{a.x / s, a.y / s, a.z / s}; }
-__device__ __forceinline__ float dot(f3 a, f3 b) { return a.x * b.x + a.y * b.y + a.z * b.z; }
+// The additions are fused by hand, a.y b.y first: left to the compiler, the order
+// of the fused additions follows the surrounding code, and with it the last
+// bit of every path.
+__device__ __forceinline__ float dot(f3 a, f3 b) {
+    return __builtin_fmaf(a.z, b.z, __builtin_fmaf(a.x, b.x, a.y * b.y));
+}
+// dot with the first two additions in the other order (exits and lenses).
+__device__ __forceinline__ float dot_xy(f3 a, f3 b) {
+    return __builtin_fmaf(a.z, b.z, __builtin_fmaf(a.y, b.y, a.x * b.x));
+}
 __device__ __forceinline__ f3 cross(f3 a, f3 b) {
     return f3{a.y * b.z - a.z * b.y, a.z * b.x - a.x * b.z, a.x * b.y - a.y * b.x};
 }
@@ -75,6 +84,19 @@ __device__ __forceinline__ void comp_add(float &hi, float &lo, float d) {
     const float s = hi + y;
     lo = y - (s - hi);
     hi = s;
+}
+
+// comp_add of the product a b, its first addition fused.
+__device__ __forceinline__ void comp_fma(float &hi, float &lo, float a, float b) {
+    const float y = __builtin_fmaf(a, b, lo);
+    const float s = hi + y;
+    lo = y - (s - hi);
+    hi = s;
+}
+
+// a + s b, fused.
+__device__ __forceinline__ f3 fma3(float s, f3 b, f3 a) {
+    return f3{__builtin_fmaf(s, b.x, a.x), __builtin_fmaf(s, b.y, a.y), __builtin_fmaf(s, b.z, a.z)};
 }
 
 }  // namespace simpler

@@ -21,6 +21,7 @@ namespace simpler {
 struct DevScene {
     f3 blockL, blockR;
     f3 inL, inR;  // blockL - eps, blockR + eps (rounded from double): the inside test's bounds
+    float ord_lo, ord_hi;  // inside the block in x and not outside the gap planes
     float ior;
     // source
     f3 light_origin;
@@ -180,6 +181,68 @@ __device__ __forceinline__ void bessel_eval(const DevScene &S, const FieldP &F, 
     }
     bessel_tab(F, F.k_r * r, J, dJ);
     if (!clamp) n = S.n_o + A * J * cm;
+    const float cr = (A * F.k_r) * dJ * ir * cm;
+    if (MM == 0) {
+        if (GA == 2)
+            g = mk3(cr * rho.x, cr * rho.y, 0.f);
+        else
+            g = general ? cr * rho : mk3(0.f, cr * rho.y, cr * rho.z);
+        return;
+    }
+    const float ctan = A * J * (float)mode * sm * ir * ir;
+    if (GA == 2) {
+        g = mk3(cr * rho.x + ctan * rho.y, cr * rho.y - ctan * rho.x, 0.f);
+    } else if (general) {
+        const f3 tp = cross(S.uz, rho);
+        g = mk3(cr * rho.x - ctan * tp.x, cr * rho.y - ctan * tp.y, cr * rho.z - ctan * tp.z);
+    } else {
+        g = mk3(0.f, cr * rho.y - ctan * rho.z, cr * rho.z + ctan * rho.y);
+    }
+}
+
+// bessel_eval at a point away from the axis (r2, the square of the distance
+// from the axis, above kBesselFarR2 > kEps^2) for the amplitude A (0 outside
+// the gap planes): the same expressions without the clamped branch.
+constexpr float kBesselFarR2 = 2e-14f;
+
+template <int GA>
+__device__ __forceinline__ void bessel_rho(const DevScene &S, f3 p, f3 &rho, float &r2) {
+    if (GA == 2) {
+        rho = mk3(p.x - S.pu.x, p.y - S.pu.y, 0.f);
+        r2 = rho.x * rho.x + rho.y * rho.y;
+    } else {
+        const f3 q = p - S.pu;
+        const float t = dot(q, S.uz);
+        rho = q - t * S.uz;
+        r2 = dot(rho, rho);
+    }
+}
+
+template <int MM, int GA>
+__device__ __forceinline__ void bessel_eval_far(const DevScene &S, const FieldP &F, f3 rho, float r2, float A, float &n,
+                                                f3 &g) {
+    const int mode = MM >= 0 ? MM : F.mode;
+    const bool general = GA >= 0 ? (GA != 0) : (S.general_axis != 0);
+    const float ir = __builtin_amdgcn_rsqf(r2);
+    const float r = r2 * ir;
+    float cm = 1.0f, sm = 0.0f;
+    if (MM != 0) {
+        const float c1 = (GA == 2 ? rho.x : dot(rho, S.ux)) * ir;
+        const float s1 = (GA == 2 ? rho.y : dot(rho, S.uy)) * ir;
+        if (MM > 0) {
+            cm = c1;
+            sm = s1;
+        }
+#pragma unroll
+        for (int k = MM > 0 ? 1 : 0; k < (MM >= 0 ? MM : mode); ++k) {
+            const float cn = cm * c1 - sm * s1;
+            sm = sm * c1 + cm * s1;
+            cm = cn;
+        }
+    }
+    float J, dJ;
+    bessel_tab(F, F.k_r * r, J, dJ);
+    n = S.n_o + A * J * cm;
     const float cr = (A * F.k_r) * dJ * ir * cm;
     if (MM == 0) {
         if (GA == 2)

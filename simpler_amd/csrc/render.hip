@@ -209,7 +209,7 @@ struct Lane {
     // number of entries held (LDS)
     float4 *q = nullptr;
     uint32_t qcap = 0;
-    volatile uint32_t *qn = nullptr;
+    uint32_t *qn = nullptr;
     int cfg = 0;  // batched renders: the photon's configuration
 };
 
@@ -320,14 +320,14 @@ __device__ __forceinline__ bool march_step(Hot &h, uint32_t &steps_left, const D
                                            float Lcut, SplineCell *cell = nullptr) {
     const float hs = h.h;
     const float hh = 0.5f * hs;
-    const f3 dvh = h.dv + hh * h.g0;
+    const f3 dvh = fma3(hh, h.g0, h.dv);
     const f3 vh = h.v + dvh;
     const float hn = hs * __builtin_amdgcn_rcpf(h.n0);
     float px = h.p.x, py = h.p.y, pz = h.p.z;
     float lx = h.pl.x, ly = h.pl.y, lz = h.pl.z;
-    comp_add(px, lx, hn * vh.x);
-    comp_add(py, ly, hn * vh.y);
-    comp_add(pz, lz, hn * vh.z);
+    comp_fma(px, lx, hn, vh.x);
+    comp_fma(py, ly, hn, vh.y);
+    comp_fma(pz, lz, hn, vh.z);
     const f3 p1 = mk3(px, py, pz);
     float n1;
     f3 g1;
@@ -337,7 +337,7 @@ __device__ __forceinline__ bool march_step(Hot &h, uint32_t &steps_left, const D
         spline_eval_cached(S, F, p1, n1, g1, *cell);
     else
         field_eval<FIELD>(S, F, p1, h.scaling, h.tau, n1, g1);
-    const f3 dv1 = dvh + hh * g1;
+    const f3 dv1 = fma3(hh, g1, dvh);
     if (COUNT) ++h.steps;
     const int lev = S.precision - h.prec;
     const bool reject = !inside_block(S, p1) || (h.travelled + hs) > h.seg_dist;
@@ -361,7 +361,7 @@ __device__ __forceinline__ bool march_step(Hot &h, uint32_t &steps_left, const D
     }
     {
         h.travelled += hs;
-        comp_add(h.L, h.Ll, hs * n1);  // optical length (scene.cpp:416)
+        comp_fma(h.L, h.Ll, hs, n1);  // optical length (scene.cpp:416)
         if (LOG) {
             if (lev == 0)
                 ++h.fcnt0;
@@ -380,6 +380,215 @@ __device__ __forceinline__ bool march_step(Hot &h, uint32_t &steps_left, const D
         }
     }
     return false;
+}
+
+// The lanes of the wave whose point p is outside the block or the gap planes.
+__device__ __forceinline__ unsigned long long not_ordinary(const DevScene &S, f3 p) {
+    return __builtin_amdgcn_ballot_w64(!(p.x >= S.ord_lo)) | __builtin_amdgcn_ballot_w64(!(p.x <= S.ord_hi)) |
+           __builtin_amdgcn_ballot_w64(!(p.y > S.inL.y)) | __builtin_amdgcn_ballot_w64(!(p.y < S.inR.y)) |
+           __builtin_amdgcn_ballot_w64(!(p.z > S.inL.z)) | __builtin_amdgcn_ballot_w64(!(p.z < S.inR.z));
+}
+
+constexpr int kFewLanes = 20;  // marching lanes of a wave up to which ordinary steps get a loop of their own
+
+// One ordinary march step (see march_chunk) of the lanes of a wave: false, and
+// nothing changed, when some lane's step is not certain to be one.
+template <int FIELD, bool LOG, int MM, int GA, bool CELL>
+__device__ __forceinline__ bool march_plain(Hot &h, const DevScene &S, const FieldP &F, SplineCell *cell) {
+    const float hs = h.h;
+    const float hh = 0.5f * hs;
+    const float hn = hs * __builtin_amdgcn_rcpf(h.n0);
+    f3 dvh = fma3(hh, h.g0, h.dv);
+    if (GA == 2) dvh.z = 0.f;
+    const f3 vh = mk3(h.v.x + dvh.x, h.v.y + dvh.y, GA == 2 ? h.v.z : h.v.z + dvh.z);
+    float px = h.p.x, py = h.p.y, pz = h.p.z;
+    float lx = h.pl.x, ly = h.pl.y, lz = h.pl.z;
+    comp_fma(px, lx, hn, vh.x);
+    comp_fma(py, ly, hn, vh.y);
+    comp_fma(pz, lz, hn, vh.z);
+    const f3 p1 = mk3(px, py, pz);
+    const float trav = h.travelled + hs;
+    unsigned long long special = not_ordinary(S, p1) | __builtin_amdgcn_ballot_w64(trav > h.seg_dist);
+    f3 rho = mk3(0.f, 0.f, 0.f);
+    float r2 = 0.f;
+    if constexpr (FIELD == kBessel) {
+        bessel_rho<GA>(S, p1, rho, r2);
+        special |= __builtin_amdgcn_ballot_w64(!(r2 > kBesselFarR2));
+    }
+    if (special) return false;
+    float n1;
+    f3 g1;
+    if constexpr (FIELD == kBessel)
+        bessel_eval_far<MM, GA>(S, F, rho, r2, F.amp * h.scaling, n1, g1);
+    else if constexpr (FIELD == kSpline && CELL)
+        spline_eval_cached(S, F, p1, n1, g1, *cell);
+    else
+        field_eval<FIELD>(S, F, p1, h.scaling, h.tau, n1, g1);
+    h.p = p1;
+    h.pl = mk3(lx, ly, lz);
+    const float dvz = h.dv.z;
+    h.dv = fma3(hh, g1, dvh);
+    if (GA == 2) h.dv.z = dvz;
+    h.n0 = n1;
+    h.g0 = g1;
+    h.travelled = trav;
+    comp_fma(h.L, h.Ll, hs, n1);
+    if (LOG) {
+        const int lev = S.precision - h.prec;
+        if (lev == 0)
+            ++h.fcnt0;
+        else
+            h.fpat += 1u << (4 * (lev - 1));
+    }
+    return true;
+}
+
+// One march step of the lanes with m set (see march_chunk); m is cleared where
+// a segment ends.  Only those lanes call it.
+template <int FIELD, bool LOG, int MM, int GA, bool CELL>
+__device__ __forceinline__ void march_masked(Hot &h, uint32_t &steps_left, bool &m, const DevScene &S, const FieldP &F,
+                                             float Lcut, SplineCell *cell) {
+    const float hs = h.h;
+    const float hh = 0.5f * hs;
+    // in the axis frame (GA 2) grad n has no z component and dv.z stays 0
+    f3 dvh = fma3(hh, h.g0, h.dv);
+    if (GA == 2) dvh.z = 0.f;
+    const f3 vh = mk3(h.v.x + dvh.x, h.v.y + dvh.y, GA == 2 ? h.v.z : h.v.z + dvh.z);
+    const float hn = hs * __builtin_amdgcn_rcpf(h.n0);
+    float px = h.p.x, py = h.p.y, pz = h.p.z;
+    float lx = h.pl.x, ly = h.pl.y, lz = h.pl.z;
+    comp_fma(px, lx, hn, vh.x);
+    comp_fma(py, ly, hn, vh.y);
+    comp_fma(pz, lz, hn, vh.z);
+    const f3 p1 = mk3(px, py, pz);
+    unsigned long long special =
+        not_ordinary(S, p1) | __builtin_amdgcn_ballot_w64((h.travelled + hs) > h.seg_dist);
+    f3 rho = mk3(0.f, 0.f, 0.f);
+    float r2 = 0.f;
+    if constexpr (FIELD == kBessel) {
+        bessel_rho<GA>(S, p1, rho, r2);
+        special |= __builtin_amdgcn_ballot_w64(!(r2 > kBesselFarR2));
+    }
+    bool act = true, acc = true;  // the step is kept; and counts as accepted
+    float n1 = 0.f;
+    f3 g1 = mk3(0.f, 0.f, 0.f);
+    if (special) {
+        const int lev = S.precision - h.prec;
+        acc = inside_block(S, p1) && !((h.travelled + hs) > h.seg_dist);
+        const bool stop = !acc && (--h.prec < 0);
+        act = acc || stop;
+        if (!act) {
+            h.h = div10(hs);
+            steps_left = 10;
+        }
+        if (LOG && stop) h.fpat |= ((uint32_t)lev << 28) | (1u << 31);
+        if constexpr (FIELD == kBessel)
+            bessel_eval<MM, GA>(S, F, p1, h.scaling, n1, g1);
+    } else {
+        if constexpr (FIELD == kBessel) bessel_eval_far<MM, GA>(S, F, rho, r2, F.amp * h.scaling, n1, g1);
+    }
+    bool fin = false;
+    if (act) {
+        if constexpr (FIELD == kSpline && CELL)
+            spline_eval_cached(S, F, p1, n1, g1, *cell);
+        else if constexpr (FIELD != kBessel)
+            field_eval<FIELD>(S, F, p1, h.scaling, h.tau, n1, g1);
+        h.p = p1;
+        h.pl = mk3(lx, ly, lz);
+        const float dvz = h.dv.z;
+        h.dv = fma3(hh, g1, dvh);
+        if (GA == 2) h.dv.z = dvz;
+        h.n0 = n1;
+        h.g0 = g1;
+        fin = !acc;
+        if (acc) {
+            h.travelled += hs;
+            comp_fma(h.L, h.Ll, hs, n1);  // optical length (scene.cpp:416)
+            if (LOG) {
+                const int lev = S.precision - h.prec;
+                if (lev == 0)
+                    ++h.fcnt0;
+                else
+                    h.fpat += 1u << (4 * (lev - 1));
+            }
+            fin = h.L > Lcut || --steps_left == 0;
+        }
+    }
+    if (__builtin_amdgcn_ballot_w64(fin)) {
+        if (fin) {
+            if (acc) {
+                h.dead = h.L > Lcut;
+                if (LOG && !h.dead) h.fpat |= (uint32_t)(S.precision - h.prec) << 28;
+            }
+            end_segment(h);
+            m = false;
+        }
+    }
+}
+
+// Up to n march steps for the lanes of the wave with m set (cleared where a
+// segment ends); adds the lane-steps taken to wave_steps.
+//
+// Nearly every step is an ordinary one: it ends inside the block, between the
+// gap planes, within the segment's distance and (Bessel) away from the axis.
+// The tests of march_step that tell these cases apart and its refinement are
+// behind one branch that the wave takes only when some lane's step is not
+// ordinary, as is the end of a segment; the rest is straight-line code
+// (march_masked).  The expressions are march_step's.  A wave with few marching
+// lanes meets such a step rarely and runs the ordinary ones in a loop of their
+// own, without masks: Bessel fields only, whose step is short enough for the
+// masks to count; with many lanes the turns between the two loops cost more.
+template <int FIELD, bool LOG, int MM, int GA, bool CELL>
+__device__ __forceinline__ void march_chunk(Hot &h, uint32_t &steps_left, bool &m, int n, const DevScene &S,
+                                            const FieldP &F, float Lcut, SplineCell *cell,
+                                            unsigned long long &wave_steps) {
+    if (FIELD == kBessel && __popcll(__builtin_amdgcn_ballot_w64(m)) <= kFewLanes) {
+        while (n > 0) {
+            const unsigned long long mm = __builtin_amdgcn_ballot_w64(m);
+            if (mm == 0ull) break;
+            int left = n;  // uniform over the marching lanes
+            if (m) {
+                // a segment's last step by its step budget leaves `left` at last
+                const int last = steps_left <= (uint32_t)n ? n - (int)steps_left : -1;
+                bool plain;
+                while (true) {
+                    plain = march_plain<FIELD, LOG, MM, GA, CELL>(h, S, F, cell);
+                    if (!plain) break;
+                    --left;
+                    if (__builtin_amdgcn_ballot_w64(h.L > Lcut) | __builtin_amdgcn_ballot_w64(left == last)) break;
+                    if (left == 0) break;
+                    // two steps per turn: the state alternates between two
+                    // sets of registers instead of being copied
+                    plain = march_plain<FIELD, LOG, MM, GA, CELL>(h, S, F, cell);
+                    if (!plain) break;
+                    --left;
+                    if (__builtin_amdgcn_ballot_w64(h.L > Lcut) | __builtin_amdgcn_ballot_w64(left == last)) break;
+                    if (left == 0) break;
+                }
+                steps_left -= (uint32_t)(n - left);
+                if (!plain) {
+                    --left;
+                    march_masked<FIELD, LOG, MM, GA, CELL>(h, steps_left, m, S, F, Lcut, cell);
+                } else {
+                    const bool over = h.L > Lcut;
+                    if (over || steps_left == 0) {
+                        h.dead = over;
+                        if (LOG && !over) h.fpat |= (uint32_t)(S.precision - h.prec) << 28;
+                        end_segment(h);
+                        m = false;
+                    }
+                }
+            }
+            left = __builtin_amdgcn_readlane(left, __ffsll((long long)mm) - 1);
+            wave_steps += (unsigned long long)__popcll(mm) * (uint32_t)(n - left);
+            n = left;
+        }
+        return;
+    }
+    for (int k = 0; k < n; ++k) {
+        wave_steps += (unsigned long long)__popcll(__builtin_amdgcn_ballot_w64(m));
+        if (m) march_masked<FIELD, LOG, MM, GA, CELL>(h, steps_left, m, S, F, Lcut, cell);
+    }
 }
 
 // march_step with the tangents of the step (forward mode; the reference's
@@ -634,8 +843,9 @@ __device__ __forceinline__ bool lens_deflect(float ap2, float f, f3 &pos, f3 &di
     dir.x = -f;
     dir.y = dir.y * invd * f - pos.y;
     dir.z = dir.z * invd * f - pos.z;
-    total += f * invd - len(dir);
-    dir = normalized(dir);
+    const float l = sqrtf(dot_xy(dir, dir));
+    total += f * invd - l;
+    dir = dir / l;
     return true;
 }
 
@@ -648,7 +858,7 @@ __device__ __forceinline__ bool exit_to_sensor(const DevScene &S, f3 &p, f3 d, f
     fw = 1.f;
     if (ior > 1.f) {
         refr.x = refr.x / ior;
-        refr = normalized(refr);
+        refr = refr / sqrtf(dot_xy(refr, refr));
         if (S.use_fresnel) fw = (1.f - fresnel_dielectric(dts.x, refr.x, 1.f / ior)) / ior / ior;
     }
     fore = dot(refr, S.cam_dir) / dot(dts, S.cam_dir);
@@ -864,15 +1074,23 @@ __device__ __forceinline__ bool nee_skip(const Lane &L, f3 d) {
 // configurations and 1.04e6 photons 1448 -> 406 ms, 2^17 of the 64^3 spline
 // 529 -> 172 ms, 2^15 of 16 point sources 1.75 -> 0.22 s.
 //
+// The number of entries is a word of LDS that only the wave's lanes access.
+__device__ __forceinline__ uint32_t wave_get(uint32_t *p) {
+    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
+}
+__device__ __forceinline__ void wave_set(uint32_t *p, uint32_t v) {
+    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
+}
+
 // nee_push: called by the lanes at a vertex (any subset of the wave); false
 // when the stack is full.
 template <int FIELD>
 __device__ __forceinline__ bool nee_push(Lane &L) {
     const unsigned long long m = __ballot(1);
     const int lane = __lane_id(), leader = __ffsll((long long)m) - 1;
-    const uint32_t held = *L.qn;
+    const uint32_t held = wave_get(L.qn);
     const uint32_t i = held + (uint32_t)__popcll(m & ((1ull << lane) - 1ull));
-    if (lane == leader) *L.qn = min(held + (uint32_t)__popcll(m), L.qcap);
+    if (lane == leader) wave_set(L.qn, min(held + (uint32_t)__popcll(m), L.qcap));
     if (i >= L.qcap) return false;
     const Hot &h = L.h;
     const Cold &c = L.c;
@@ -1294,9 +1512,26 @@ static_assert(5 * (sizeof(Cold) * kBlock + sizeof(uint32_t) * (C_N + kBlock / 64
                   160 * 1024,
               "five single-scene Bessel workgroups must fit one CU's LDS");
 
+// A kernel argument at its offset of the argument segment, through a pointer
+// that the compiler takes for new at each call, so that what is read through
+// it is loaded where it is used and not kept in registers.  Read as plain
+// arguments, 150 scalars were spilled to vector registers and 45 vectors to
+// scratch in the m = 0 kernel (0 and 2 now), and the batched kernels fit three
+// waves per SIMD instead of four: 2^22 photons 447 -> 413 ms, the
+// 256-configuration sweep 391 -> 362 ms, 2^17 spline photons 172 -> 141 ms.
+template <class T>
+__device__ __forceinline__ const T &kernel_arg(size_t offset) {
+    using Segment = const __attribute__((address_space(4))) char *;
+    Segment p = (Segment)__builtin_amdgcn_kernarg_segment_ptr();
+    asm volatile("" : "+s"(p));
+    return *(const T *)(p + offset);
+}
+// k_render's arguments: a DevScene, then a RenderArgs
+constexpr size_t kArgsOffset = (sizeof(DevScene) + alignof(RenderArgs) - 1) / alignof(RenderArgs) * alignof(RenderArgs);
+
 template <int FIELD, int MODE, bool BATCH, bool JLDS = false, int MM = -1, int GA = -1, int SPLAT = 0>
 __global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(FIELD == kBessel ? 5 : (FIELD == kSpline ? 2 : 1))))
-k_render(DevScene S, RenderArgs A) {
+k_render(DevScene S0, RenderArgs A0) {
     __shared__ Cold cold[kBlock];
     __shared__ uint32_t cnt[C_N];
     __shared__ float4 jlds[JLDS ? (BATCH ? kJtabLdsBatch : 4 * kJtabLds) : 1];
@@ -1306,16 +1541,11 @@ k_render(DevScene S, RenderArgs A) {
     if (threadIdx.x < C_N) cnt[threadIdx.x] = 0u;
     if (STACK && (threadIdx.x & 63) == 0) nheld[threadIdx.x >> 6] = 0u;
     if (JLDS) {
-        const float4 *src = BATCH ? A.jtab_base : S.jtab;
-        const int nj = BATCH ? A.jtab_len : 4 * S.jtab_n;
+        const float4 *src = BATCH ? A0.jtab_base : S0.jtab;
+        const int nj = BATCH ? A0.jtab_len : 4 * S0.jtab_n;
         for (int i = threadIdx.x; i < nj; i += blockDim.x) jlds[i] = src[i];
     }
     __syncthreads();
-    Var vsingle = var_from(S, A);
-    if (JLDS && !BATCH) vsingle.f.jtab = jlds;
-    // batch: the lane's configuration, read from global memory (L1/L2
-    // resident), replaced when the lane takes a photon of another one
-    Var *vp = BATCH ? const_cast<Var *>(A.cfgs) : &vsingle;
     Hot h;
     h.steps = 0;
     h.state = ST_NEED;
@@ -1325,27 +1555,40 @@ k_render(DevScene S, RenderArgs A) {
     Tan tan;
     SplineCell scell;
     scell.key = -1;
-    Lane L{h, cold[threadIdx.x], vp, S, A, cnt, nullptr, &mcache[threadIdx.x], SPLAT ? &ps : nullptr,
-           MODE == M_JVP ? &tan : nullptr};
-    const int lane = __lane_id();
-    if (STACK) {
-        const int wave = (int)((blockIdx.x * blockDim.x + threadIdx.x) >> 6);
-        L.qn = &nheld[threadIdx.x >> 6];
-        L.qcap = __builtin_amdgcn_readfirstlane(wave < A.nq_waves ? A.nq_cap : 0);
-        L.q = A.nq + (size_t)__builtin_amdgcn_readfirstlane(wave) * A.nq_cap * kJobVec;
-    }
-    bool left = true;  // photons left in the launch's queue (uniform)
+    int cfg = 0;        // batch: the lane's configuration
+    bool left = true;   // photons left in the launch's queue (uniform)
     unsigned long long wave_steps = 0;  // ER steps of the wave (uniform)
     while (true) {
+        // The event code reads the scene, the arguments and its addresses
+        // anew on every turn: held across the march loop (about 200 scalars
+        // and a few vectors) they would fill the registers and be spilled.
+        const DevScene &S = kernel_arg<DevScene>(0);
+        const RenderArgs &A = kernel_arg<RenderArgs>(kArgsOffset);
+        int tid = (int)threadIdx.x;
+        asm volatile("" : "+v"(tid));
+        Var vsingle = var_from(S, A);
+        if (JLDS && !BATCH) vsingle.f.jtab = jlds;
+        // batch: the lane's configuration, read from global memory (L1/L2
+        // resident), replaced when the lane takes a photon of another one
+        Lane L{h, cold[tid], BATCH ? const_cast<Var *>(A.cfgs) + cfg : &vsingle, S, A, cnt, nullptr, &mcache[tid],
+               SPLAT ? &ps : nullptr, MODE == M_JVP ? &tan : nullptr};
+        const int lane = __lane_id();
+        if (STACK) {
+            const int wave = __builtin_amdgcn_readfirstlane((int)((blockIdx.x * blockDim.x + tid) >> 6));
+            L.qn = &nheld[tid >> 6];
+            L.qcap = wave < A.nq_waves ? A.nq_cap : 0;
+            L.q = A.nq + (size_t)wave * A.nq_cap * kJobVec;
+            L.cfg = cfg;
+        }
         // fetch: first the wave's next-event stack, then new photons, one
         // atomic per wave for all lanes that take one
         unsigned long long need = __ballot(h.state == ST_NEED);
         if (STACK && need) {
-            const uint32_t held = __builtin_amdgcn_readfirstlane(*L.qn);
+            const uint32_t held = __builtin_amdgcn_readfirstlane(wave_get(L.qn));
             if (held) {
                 const uint32_t want = (uint32_t)__popcll(need);
                 const uint32_t rank = (uint32_t)__popcll(need & ((1ull << lane) - 1ull));
-                if (lane == 0) *L.qn = held - min(held, want);
+                if (lane == 0) wave_set(L.qn, held - min(held, want));
                 __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
                 if (h.state == ST_NEED && rank < held) {
                     nee_pop<FIELD, BATCH>(L, held - 1u - rank);
@@ -1397,35 +1640,36 @@ k_render(DevScene S, RenderArgs A) {
         if (h.state == ST_SEG_END) seg_end<FIELD, MODE>(L);
         if (SPLAT) wave_splat(ps, A);
         if (__ballot(h.state == ST_MARCH) == 0ull) {
-            if (__ballot(h.state != ST_NEED) == 0ull && !left && (!STACK || *L.qn == 0u)) break;
+            if (__ballot(h.state != ST_NEED) == 0ull && !left && (!STACK || __builtin_amdgcn_readfirstlane(wave_get(L.qn)) == 0u)) break;
             continue;
         }
-        FieldP F = L.v->f;
-        if (BATCH && JLDS) F.jtab = jlds + (F.jtab - A.jtab_base);
-        float Lcut = L.v->Lcut;
+        if (BATCH) cfg = L.cfg;
+        FieldP F = BATCH ? L.v->f : field_params(S0);
+        if (JLDS) F.jtab = BATCH ? jlds + (F.jtab - A.jtab_base) : jlds;
+        float Lcut = BATCH ? L.v->Lcut : S0.Lcut;
         // held in a vector register through the march loop: the kernel's
         // scalar registers are full, and a scalar copy is reloaded from its
         // spill lanes on every step
         asm volatile("" : "+v"(Lcut));
         bool m = h.state == ST_MARCH;
         uint32_t sl = h.steps_left;
-        for (int k = 0; k < A.spc; ++k) {
-            wave_steps += __popcll(__ballot(m));  // one ER step per marching lane
-            if constexpr (MODE == M_JVP) {
-                if (m) m = !march_step_jvp<FIELD>(h, tan, sl, S, F, Lcut, A.theta_dot);
-            } else {
-                if (m) m = !march_step<FIELD, false, MM, false, GA, FIELD == kSpline>(h, sl, S, F, Lcut, &scell);
+        if constexpr (MODE == M_JVP) {
+            for (int k = 0; k < A0.spc; ++k) {
+                wave_steps += __popcll(__ballot(m));  // one ER step per marching lane
+                if (m) m = !march_step_jvp<FIELD>(h, tan, sl, S0, F, Lcut, A0.theta_dot);
             }
+        } else {
+            march_chunk<FIELD, false, MM, GA, FIELD == kSpline>(h, sl, m, A0.spc, S0, F, Lcut, &scell, wave_steps);
         }
         h.steps_left = sl;
         if (h.state == ST_MARCH && !m) h.state = ST_SEG_END;
     }
     // counters: ER steps reduced over the wave, events from LDS, one atomic
     // per counter per wave / block
-    if (lane == 0 && wave_steps) atomicAdd(A.counters + C_STEPS, wave_steps);
+    if (__lane_id() == 0 && wave_steps) atomicAdd(A0.counters + C_STEPS, wave_steps);
     __syncthreads();
     if (threadIdx.x < C_N && threadIdx.x != C_STEPS && cnt[threadIdx.x])
-        atomicAdd(A.counters + threadIdx.x, (unsigned long long)cnt[threadIdx.x]);
+        atomicAdd(A0.counters + threadIdx.x, (unsigned long long)cnt[threadIdx.x]);
 }
 
 __global__ void k_fill_f32(float *p, size_t n, float v) {
@@ -1811,6 +2055,10 @@ static DevScene make_dev_scene(const simpler_scene *sc, int64_t n_total, uint64_
     S.inR = f3{(float)((double)d.block_r[0] + kEps), (float)((double)d.block_r[1] + kEps),
                (float)((double)d.block_r[2] + kEps)};
     S.blockR = h3(d.block_r);
+    // the x range of march_chunk's ordinary steps: inside the block and not
+    // outside the gap planes
+    S.ord_lo = std::max(std::nextafter(S.inL.x, INFINITY), d.sgap_begin_loc_x);
+    S.ord_hi = std::min(std::nextafter(S.inR.x, -INFINITY), d.egap_end_loc_x);
     S.ior = d.ior;
     S.light_origin = h3(d.light_origin);
     S.ct = std::cos(d.half_theta_limit);
