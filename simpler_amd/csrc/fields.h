@@ -353,11 +353,13 @@ __device__ __forceinline__ void spline_row(float c0, float c1, float c2, float c
 // c, b, q from the base corner: read in place from the padded copy, or from
 // a register copy of the cell (SplineCell).
 struct PadTaps {
+    static constexpr bool kCell = false;
     const float *base;
     long row, slab;
     __device__ __forceinline__ float operator()(int c, int b, int q) const { return base[c * slab + b * row + q]; }
 };
 struct CellTaps {
+    static constexpr bool kCell = true;
     const float *t;
     __device__ __forceinline__ float operator()(int c, int b, int q) const { return t[(c * 4 + b) * 4 + q]; }
 };
@@ -369,7 +371,10 @@ __device__ __forceinline__ bool spline_padded(const DevScene &S, int jx, int jy,
            (unsigned)jz <= (unsigned)(S.sP[2] - 4);
 }
 
-// Value and gradient sums over the taps (x, then y, then z passes).
+// Value and gradient sums over the taps (x, then y, then z passes).  The
+// fused additions of a register cell's rows are written out, the first two in
+// the order that the compiler had chosen for each row: left to it, the order
+// follows the surrounding code, and kernels differ in the last bit of n.
 template <class Taps>
 __device__ __forceinline__ void spline_sum(const Taps &T, const float wx[4], const float dwx[4], const float wy[4],
                                            const float dwy[4], const float wz[4], const float dwz[4], float &v,
@@ -378,8 +383,22 @@ __device__ __forceinline__ void spline_sum(const Taps &T, const float wx[4], con
     for (int c = 0; c < 4; ++c) {
         float s0 = 0.f, sx = 0.f, sy0 = 0.f;
 #pragma unroll
-        for (int b = 0; b < 4; ++b)
-            spline_row(T(c, b, 0), T(c, b, 1), T(c, b, 2), T(c, b, 3), wx, dwx, wy[b], dwy[b], s0, sx, sy0);
+        for (int b = 0; b < 4; ++b) {
+            if constexpr (Taps::kCell) {
+                const int i = c * 4 + b < 13 ? 0 : 1, j = 1 - i;
+                const float a0 = __builtin_fmaf(
+                    T(c, b, 3), wx[3],
+                    __builtin_fmaf(T(c, b, 2), wx[2], __builtin_fmaf(T(c, b, j), wx[j], T(c, b, i) * wx[i])));
+                const float a1 = __builtin_fmaf(
+                    T(c, b, 3), dwx[3],
+                    __builtin_fmaf(T(c, b, 2), dwx[2], __builtin_fmaf(T(c, b, j), dwx[j], T(c, b, i) * dwx[i])));
+                s0 += a0 * wy[b];
+                sx += a1 * wy[b];
+                sy0 += a0 * dwy[b];
+            } else {
+                spline_row(T(c, b, 0), T(c, b, 1), T(c, b, 2), T(c, b, 3), wx, dwx, wy[b], dwy[b], s0, sx, sy0);
+            }
+        }
         v += s0 * wz[c];
         vx += sx * wz[c];
         vy += sy0 * wz[c];
