@@ -473,13 +473,15 @@ int simpler_ctx_get_splat(simpler_ctx *ctx, int *strategy);
  * that splats into the objective runs the sub-path backwards at once, and the
  * photon's main path when it ends, while the other lanes of its wave march
  * on; 1 (default) = deferred: the re-trace queues each such sub-path (its log
- * and adjoint seed) and each photon's main-path log, then a second kernel runs
- * the queued sub-paths and a third the main paths, every lane reversing.
+ * and adjoint seed) and the main-path log of each photon with a next-event
+ * sub-path, then a second kernel runs the queued sub-paths and a third the main
+ * paths, every lane reversing.
  * queue_capacity c (0 keeps the current value, default 2^23; else
  * 64 <= c <= 2^26) sizes the queues of one chunk of photons: c sub-paths
  * with c sub-path records, c main paths with 8 c main-path records, 768 c
  * bytes of device memory (6 GiB at the default), allocated on first use and
- * kept by the context.  The chunk starts at 2^22 photons, halves when a
+ * kept by the context.  The chunk starts at 2^22 photons (less where the mean
+ * path's main-path records would pass 90 % of their queue), halves when a
  * chunk's queues overflow (the chunk is then traced again) and doubles, up
  * to 2^24, after a chunk that filled no queue past 40 %; at 2^14 photons an
  * overflowing chunk runs inline.  Both schedules give the same objective

@@ -55,6 +55,11 @@ struct AdjState {
     uint32_t rcnt0, rpat;
     int rphase, rseg, nsub, nmain, last_lam;
     int slot;       // deferred re-trace: the photon's main-path slot, -1 none
+    // deferred re-trace: the current next-event sub-path's main-path slot and
+    // vertex record (the lane may have it from another lane's photon), and
+    // whether that main path's log was full
+    int jslot, jvert;
+    bool jtrunc;
     int cfg;        // batched kernels: the lane's configuration
     bool pending, trunc_main, trunc_sub;
     double F;
@@ -377,16 +382,9 @@ __device__ __forceinline__ void adj_defer_sub(Lane &L, f3 lp, f3 lv, float mu, f
     const Hot &h = L.h;
     int slot = -1;
     if (phase == RP_NEE) {
-        if (a.slot < 0) {
-            const unsigned long long sl = atomicAdd(A.qcnt + Q_SLOTS, 1ull);
-            if (sl >= A.slot_cap) {
-                adj_overflow(A);
-                return;
-            }
-            a.slot = (int)sl;
-        }
-        slot = a.slot;
-        a.last_lam = a.nmain - 1;
+        slot = a.jslot;
+        if (slot < 0) return;  // no slot left: adj_vertex_slot flagged it
+        atomicMax(reinterpret_cast<int *>(A.slots + (size_t)slot * 16 + 6), a.jvert);
     }
     const unsigned long long j = atomicAdd(A.qcnt + Q_JOBS, 1ull);
     if (j >= A.job_cap) {
@@ -409,15 +407,51 @@ __device__ __forceinline__ void adj_defer_sub(Lane &L, f3 lp, f3 lv, float mu, f
     r[3] = make_float4(lv.x, lv.y, lv.z, ln);
     r[4] = make_float4(a.ldin.x, a.ldin.y, a.ldin.z, h.scaling);
     r[5] = make_float4(L.c.mp.x, L.c.mp.y, L.c.mp.z, h.tau);
-    r[6] = make_float4(__int_as_float(slot), __int_as_float(a.nmain - 1), __int_as_float(phase),
-                       __int_as_float(a.nsub));
+    r[6] = make_float4(__int_as_float(slot), __int_as_float(a.jvert), __int_as_float(phase), __int_as_float(a.nsub));
     r[7] = make_float4(__uint_as_float((uint32_t)sb), __uint_as_float((uint32_t)(sb >> 32)), __int_as_float(a.cfg),
                        0.f);
 }
 
+// A vertex of the deferred re-trace with a next-event sub-path to trace: the
+// photon's main-path slot (taken at its first such vertex; its last vertex
+// with an adjoint starts at none) and what the sub-path's job needs to know
+// of it.
+__device__ __forceinline__ void adj_vertex_slot(Lane &L) {
+    AdjState &a = *L.a;
+    const RenderArgs &A = L.A;
+    if (a.slot < 0 && !a.trunc_main) {
+        const unsigned long long sl = atomicAdd(A.qcnt + Q_SLOTS, 1ull);
+        if (sl >= A.slot_cap) {
+            adj_overflow(A);
+        } else {
+            a.slot = (int)sl;
+            atomicExch(reinterpret_cast<int *>(A.slots + (size_t)sl * 16 + 6), -1);
+        }
+    }
+    a.jslot = a.slot;
+    a.jvert = a.nmain - 1;
+    a.jtrunc = a.trunc_main;
+}
+
+// The adjoint's part of an entry of the next-event stack.
+__device__ __forceinline__ void adj_job_store(const Lane &L, float4 *r) {
+    const AdjState &a = *L.a;
+    *r = make_float4(L.h.tau, __int_as_float(a.jslot), __int_as_float(a.jvert), __int_as_float(a.jtrunc ? 1 : 0));
+}
+__device__ __forceinline__ void adj_job_load(Lane &L, float4 r) {
+    AdjState &a = *L.a;
+    L.h.tau = r.x;
+    a.jslot = __float_as_int(r.y);
+    a.jvert = __float_as_int(r.z);
+    a.jtrunc = __float_as_int(r.w) != 0;
+    L.c.mp = L.h.p;
+    adj_sub_begin(a);
+}
+
 // Photon end of the deferred re-trace: store the main-path log of a photon
-// with queued next-event sub-paths (slot layout: source, scaling; tau,
-// record count, last vertex with an adjoint, valid; record base,
+// with traced next-event sub-paths, which may still be on the wave's stack
+// (slot layout: source, scaling; tau, record count, last vertex with an
+// adjoint -- kept by the sub-paths' jobs -- valid; record base,
 // configuration).
 __device__ __forceinline__ void adj_store_slot(Lane &L) {
     AdjState &a = *L.a;
@@ -435,7 +469,8 @@ __device__ __forceinline__ void adj_store_slot(Lane &L) {
         }
     }
     r[0] = make_float4(a.src.x, a.src.y, a.src.z, L.h.scaling);
-    r[1] = make_float4(L.h.tau, __int_as_float(a.nmain), __int_as_float(a.last_lam), __int_as_float(valid));
+    *reinterpret_cast<float2 *>(r + 1) = make_float2(L.h.tau, __int_as_float(a.nmain));
+    reinterpret_cast<int *>(r + 1)[3] = valid;
     r[2] = make_float4(__uint_as_float((uint32_t)base), __uint_as_float((uint32_t)(base >> 32)), __int_as_float(a.cfg),
                        0.f);
 }
@@ -465,6 +500,11 @@ __device__ __forceinline__ void sub_rev_start(Lane &L, f3 lp, f3 lv, float mu, f
     rev_init(h, a, S.h0, h.fcnt0, h.fpat);
 }
 
+// The objective weights of the lane's configuration.
+__device__ __forceinline__ const float *adj_weights(const Lane &L) {
+    return L.A.G + (size_t)L.a->cfg * L.A.X * L.A.Y * L.A.Z;
+}
+
 // NEE splat (scene.cpp:897-929) differentiated:
 //   val = W 2 pi exp(-sigma d) f_HG(din . dts) fore fw,
 //   fore = (refr . c) / (dts . c); fw (Fresnel transmission) is held fixed.
@@ -476,9 +516,9 @@ __device__ __forceinline__ bool nee_adj_start(Lane &L, f3 ps, float Lv, float va
     const DevScene &S = L.S;
     float Wsum;
     f3 lps;
-    if (!splat_adj(S, L.A, L.v->image, ps, Lv, L.c.depth, val, Wsum, lps)) return false;
+    if (!splat_adj(S, L.A, adj_weights(L), ps, Lv, L.c.depth, val, Wsum, lps)) return false;
     a.F += (double)val * (double)Wsum;
-    if (a.trunc_sub || a.trunc_main) {
+    if (a.trunc_sub || (DEFER ? a.jtrunc : a.trunc_main)) {
         ++a.dropped;
         return false;
     }
@@ -511,7 +551,7 @@ __device__ __forceinline__ bool direct_adj_start(Lane &L, f3 ps, float Lv, float
     const DevScene &S = L.S;
     float Wsum;
     f3 lps;
-    if (!splat_adj(S, L.A, L.v->image, ps, Lv, 0, val, Wsum, lps)) return false;
+    if (!splat_adj(S, L.A, adj_weights(L), ps, Lv, 0, val, Wsum, lps)) return false;
     a.F += (double)val * (double)Wsum;
     if (a.trunc_sub) {
         ++a.dropped;

@@ -141,30 +141,20 @@ __device__ __forceinline__ void adj_flush_cfg(AdjState &a, const RenderArgs &A, 
 // loop plus the backward events (ST_REND, ST_MREV) and backward steps.
 // BATCH: photons of many point-source patterns (per-pattern amplitudes,
 // phases, photon budget, seed, objective weights, gradient and objective).
-// M_ADJDEF: the deferred image adjoint's re-trace: forward runs and logs
-// only, backward runs queued for k_adj_rev (no parameter derivatives here).
-// The spline re-trace is held to 256 registers (2 waves per SIMD, as the
-// spline render); it needs a few more, which spill.
 template <int FIELD, int MODE, bool BATCH = false>
-__global__ void __launch_bounds__(kBlock)
-    __attribute__((amdgpu_waves_per_eu(MODE == M_ADJDEF && FIELD == kSpline ? 2 : 1)))
-    k_adjoint(DevScene S, RenderArgs A) {
-    constexpr bool DEF = MODE == M_ADJDEF;
+__global__ void __launch_bounds__(kBlock) k_adjoint(DevScene S, RenderArgs A) {
     __shared__ Cold cold[kBlock];
     __shared__ uint32_t cnt[C_N];
-    __shared__ float sacc[DEF ? 1
-                              : (FIELD == kSources ? (2 * kMaxAdjSources + 1) * kBlock
-                                                   : (FIELD == kBessel ? 3 * kBlock : 1))];
-    __shared__ float vcell[FIELD == kSpline && !DEF ? 64 * kBlock : 1];  // spline VJP cell sums
-    if (FIELD == kSpline && !DEF)
+    __shared__ float sacc[FIELD == kSources ? (2 * kMaxAdjSources + 1) * kBlock : (FIELD == kBessel ? 3 * kBlock : 1)];
+    __shared__ float vcell[FIELD == kSpline ? 64 * kBlock : 1];  // spline VJP cell sums
+    if (FIELD == kSpline)
         for (int t = 0; t < 64; ++t) vcell[t * kBlock + threadIdx.x] = 0.f;
     __shared__ Var vars[BATCH ? kBlock : 1];
     if (threadIdx.x < C_N) cnt[threadIdx.x] = 0u;
-    const int npar = DEF ? 0 : (FIELD == kSources ? 2 * S.n_src + 1 : (FIELD == kBessel ? 3 : 0));
+    const int npar = FIELD == kSources ? 2 * S.n_src + 1 : (FIELD == kBessel ? 3 : 0);
     for (int j = 0; j < npar; ++j) sacc[j * kBlock + threadIdx.x] = 0.f;
     __syncthreads();
     Var vsingle = var_from(S, A);
-    vsingle.image = const_cast<float *>(A.G);  // the objective weights, read by the splat adjoint
     Var &v = BATCH ? vars[threadIdx.x] : vsingle;
     int cur_cfg = -1;
     Hot h;
@@ -186,7 +176,7 @@ __global__ void __launch_bounds__(kBlock)
     a.G.grid = FIELD == kSpline && A.gx ? A.gx + (size_t)xcd_id() * A.gx_stride : A.grad;
     a.G.acc = sacc + threadIdx.x;
     a.G.stride = kBlock;
-    a.G.cell = FIELD == kSpline && !DEF ? vcell + threadIdx.x : nullptr;
+    a.G.cell = FIELD == kSpline ? vcell + threadIdx.x : nullptr;
     a.G.kx = -1;
     Lane L{h, cold[threadIdx.x], &v, S, A, cnt, &a, nullptr, nullptr, nullptr, true};
     const int lane = __lane_id();
@@ -204,7 +194,7 @@ __global__ void __launch_bounds__(kBlock)
                     uint64_t pid = A.offset + idx;
                     if (BATCH) {
                         // the photon's index over all configurations (A.offset:
-                        // the start of a deferred chunk)
+                        // the start of a chunk)
                         const unsigned long long gi = A.offset + idx;
                         int lo = 0, hi = A.n_cfg;  // largest c with prefix[c] <= gi
                         while (hi - lo > 1) {
@@ -220,7 +210,6 @@ __global__ void __launch_bounds__(kBlock)
                             cur_cfg = lo;
                             a.cfg = lo;
                             v = A.cfgs[lo];
-                            v.image = const_cast<float *>(A.G) + (size_t)lo * A.X * A.Y * A.Z;
                         }
                     }
                     L.c.pid_lo = (uint32_t)pid;
@@ -233,15 +222,8 @@ __global__ void __launch_bounds__(kBlock)
         }
         if (h.state == ST_INIT) photon_init<FIELD, MODE>(L);
         if (h.state == ST_SEG_END) seg_end<FIELD, MODE>(L);
-        if constexpr (DEF) {  // a photon with queued next-event sub-paths ended: store its main path
-            if (h.state == ST_NEED && a.slot >= 0) {
-                adj_store_slot(L);
-                a.slot = -1;
-            }
-        } else {
-            if (h.state == ST_REND) rev_end<FIELD, MODE>(L);
-            if (h.state == ST_MREV) main_rev_init<FIELD>(L);
-        }
+        if (h.state == ST_REND) rev_end<FIELD, MODE>(L);
+        if (h.state == ST_MREV) main_rev_init<FIELD>(L);
         if (__ballot(h.state != ST_DONE) == 0ull) break;
         if (__ballot(h.state == ST_MARCH || h.state == ST_RMARCH) == 0ull) continue;
         const FieldP F = v.f;
@@ -251,7 +233,7 @@ __global__ void __launch_bounds__(kBlock)
         for (int k = 0; k < A.spc; ++k) {
             if (m)
                 m = !march_step<FIELD, true, -1, true, -1, FIELD == kSpline>(h, sl, S, F, Lcut, &scell);
-            else if (!DEF && r)
+            else if (r)
                 r = rev_step<FIELD, FIELD == kSpline>(h, a, S, F, &scell);
         }
         h.steps_left = sl;
@@ -259,7 +241,7 @@ __global__ void __launch_bounds__(kBlock)
         if (h.state == ST_RMARCH && !r) h.state = ST_REND;
     }
     if (BATCH) adj_flush_cfg(a, A, cur_cfg, npar);
-    if (FIELD == kSpline && !DEF) spline_cell_flush(S, a.G);
+    if (FIELD == kSpline) spline_cell_flush(S, a.G);
     unsigned long long st = h.steps;
     double fo = a.F;
     unsigned long long ac[A_N] = {a.rsteps, a.nsubrev, a.nmainrev, a.dropped};
@@ -284,6 +266,147 @@ __global__ void __launch_bounds__(kBlock)
         for (int t = 0; t < kBlock; ++t) sum += sacc[j * kBlock + t];
         if (sum != 0.f) atomicAdd(A.grad + j, sum);
     }
+}
+
+// The deferred image adjoint's re-trace: forward runs and logs only, backward
+// runs queued for k_adj_rev (no parameter derivatives here).  The render
+// kernel's loop: next-event sub-paths on the wave's stack, march_chunk, the
+// event code's arguments re-read on every turn.  BATCH: photons of many
+// point-source patterns; a lane's objective sum goes to its pattern's when
+// the lane moves to another one.
+// A small launch is bound by the chain of its longest photon; before, that was
+// the main path and all its sub-paths, one lane per photon.  Whole adjoint,
+// before -> with this and the spread backward kernels: 2^17 photons of the
+// 64^3 spline scene 427 -> 211 ms, 64 patterns of 2,048 photons 1043 -> 529 ms.
+template <int FIELD, bool BATCH = false>
+__global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(FIELD == kSpline ? 2 : 1)))
+k_retrace(DevScene S0, RenderArgs A0) {
+    constexpr int MODE = M_ADJDEF;
+    __shared__ Cold cold[kBlock];
+    __shared__ uint32_t cnt[C_N];
+    __shared__ uint32_t nheld[kBlock / 64];  // entries of each wave's next-event stack
+    if (threadIdx.x < C_N) cnt[threadIdx.x] = 0u;
+    if ((threadIdx.x & 63) == 0) nheld[threadIdx.x >> 6] = 0u;
+    __syncthreads();
+    Hot h;
+    h.steps = 0;
+    h.state = ST_NEED;
+    h.dead = false;
+    AdjState a;
+    SplineCell scell;  // spline kernels: register copy of the current cell's taps
+    scell.key = -1;
+    a.F = 0.0;
+    a.rsteps = a.nsubrev = a.nmainrev = a.dropped = 0;
+    a.pending = a.trunc_main = a.trunc_sub = a.jtrunc = false;
+    a.slot = a.jslot = -1;
+    a.cfg = 0;
+    a.gL = 0.f;
+    bool left = true;  // photons left in the launch's queue (uniform)
+    unsigned long long wave_steps = 0;  // ER steps of the wave (uniform)
+    while (true) {
+        const DevScene &S = kernel_arg<DevScene>(0);
+        const RenderArgs &A = kernel_arg<RenderArgs>(kArgsOffset);
+        int tid = (int)threadIdx.x;
+        asm volatile("" : "+v"(tid));
+        Var vsingle = var_from(S, A);
+        Lane L{h, cold[tid], BATCH ? const_cast<Var *>(A.cfgs) + a.cfg : &vsingle, S, A, cnt, &a, nullptr, nullptr,
+               nullptr, true};
+        const size_t gid = (size_t)blockIdx.x * kBlock + tid;
+        a.log_main = A.log + gid * (size_t)(A.main_cap + A.sub_cap) * kRecFloats;
+        a.log_sub = a.log_main + (size_t)A.main_cap * kRecFloats;
+        const int lane = __lane_id();
+        const int wave = __builtin_amdgcn_readfirstlane((int)(gid >> 6));
+        L.qn = &nheld[tid >> 6];
+        L.qcap = wave < A.nq_waves ? A.nq_cap : 0;
+        L.q = A.nq + (size_t)wave * A.nq_cap * job_vec(MODE);
+        L.cfg = a.cfg;
+        // the lane's objective to its configuration's, before it takes
+        // another one's work
+        auto set_cfg = [&](int c) {
+            if (BATCH && c != a.cfg) {
+                if (a.F != 0.0) atomicAdd(A.obj + a.cfg, a.F);
+                a.F = 0.0;
+                a.cfg = L.cfg = c;
+                L.v = const_cast<Var *>(A.cfgs) + c;
+            }
+        };
+        unsigned long long need = __ballot(h.state == ST_NEED);
+        if (need) {
+            const uint32_t held = __builtin_amdgcn_readfirstlane(wave_get(L.qn));
+            if (held) {
+                const uint32_t want = (uint32_t)__popcll(need);
+                const uint32_t rank = (uint32_t)__popcll(need & ((1ull << lane) - 1ull));
+                if (lane == 0) wave_set(L.qn, held - min(held, want));
+                __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+                if (h.state == ST_NEED && rank < held) {
+                    const uint32_t i = held - 1u - rank;
+                    if (BATCH) set_cfg(__float_as_int(L.q[(size_t)i * job_vec(MODE) + 3].w));
+                    nee_pop<FIELD, MODE, false>(L, i);
+                }
+                need = __ballot(h.state == ST_NEED && rank >= held);
+            }
+        }
+        if (need && left && A.wave_photons < 64) {  // fewer photons than lanes: spread over the waves
+            const int mains = __popcll(__ballot(h.state != ST_NEED && L.c.phase != PH_JOB));
+            const int room = max(A.wave_photons - mains, 0);
+            while (__popcll(need) > room) need &= need - 1ull;
+        }
+        if (need && left) {
+            const unsigned long long base = wave_take(A.work, need);
+            left = base + __popcll(need) < A.n;
+            if ((need >> lane) & 1ull) {
+                const unsigned long long idx = base + __popcll(need & ((1ull << lane) - 1ull));
+                if (idx < A.n) {
+                    uint64_t pid = A.offset + idx;
+                    if (BATCH) {  // A.offset + idx: the photon's index over all configurations
+                        int c;
+                        pid = batch_photon(A, A.offset + idx, c);
+                        set_cfg(c);
+                    }
+                    L.c.pid_lo = (uint32_t)pid;
+                    L.c.pid_hi = (uint32_t)(pid >> 32);
+                    h.state = ST_INIT;
+                }
+            }
+        }
+        if (h.state == ST_INIT) photon_init<FIELD, MODE>(L);
+        if (h.state == ST_SEG_END) seg_end<FIELD, MODE>(L);
+        if (h.state == ST_NEED && a.slot >= 0) {  // a photon with traced next-event sub-paths ended
+            adj_store_slot(L);
+            a.slot = -1;
+        }
+        if (__ballot(h.state == ST_MARCH) == 0ull) {
+            if (__ballot(h.state != ST_NEED) == 0ull && !left && __builtin_amdgcn_readfirstlane(wave_get(L.qn)) == 0u)
+                break;
+            continue;
+        }
+        const FieldP F = BATCH ? L.v->f : field_params(S0);
+        float Lcut = BATCH ? L.v->Lcut : S0.Lcut;
+        asm volatile("" : "+v"(Lcut));
+        bool m = h.state == ST_MARCH;
+        uint32_t sl = h.steps_left;
+        march_chunk<FIELD, true, -1, -1, FIELD == kSpline>(h, sl, m, A0.spc, S0, F, Lcut, &scell, wave_steps);
+        h.steps_left = sl;
+        if (h.state == ST_MARCH && !m) h.state = ST_SEG_END;
+    }
+    double fo = a.F;
+    unsigned long long dropped = a.dropped;
+    if (BATCH) {
+        if (fo != 0.0) atomicAdd(A0.obj + a.cfg, fo);
+        fo = 0.0;
+    }
+    for (int off = 32; off > 0; off >>= 1) {
+        fo += __shfl_xor(fo, off);
+        dropped += __shfl_xor(dropped, off);
+    }
+    if (__lane_id() == 0) {
+        if (wave_steps) atomicAdd(A0.counters + C_STEPS, wave_steps);
+        if (fo != 0.0) atomicAdd(A0.obj, fo);
+        if (dropped) atomicAdd(A0.acnt + A_DROPPED, dropped);
+    }
+    __syncthreads();
+    if (threadIdx.x < C_N && threadIdx.x != C_STEPS && cnt[threadIdx.x])
+        atomicAdd(A0.counters + threadIdx.x, (unsigned long long)cnt[threadIdx.x]);
 }
 
 // The configuration of a queued job or stored slot (batched adjoint).
@@ -331,7 +454,8 @@ __device__ __forceinline__ void job_load(Lane &L, unsigned long long j) {
 }
 
 // A stored main path (adj_store_slot's layout) as the lane's backward run;
-// false for a photon whose log was not stored.
+// false for a photon whose log was not stored or whose sub-paths all missed
+// the objective.
 template <int FIELD>
 __device__ __forceinline__ bool slot_load(Lane &L, unsigned long long s) {
     AdjState &a = *L.a;
@@ -339,7 +463,7 @@ __device__ __forceinline__ bool slot_load(Lane &L, unsigned long long s) {
     const RenderArgs &A = L.A;
     const float4 *r = reinterpret_cast<const float4 *>(A.slots + s * 16);
     const float4 r0 = r[0], r1 = r[1], r2 = r[2];
-    if (!__float_as_int(r1.w)) return false;
+    if (!__float_as_int(r1.w) || __float_as_int(r1.z) < 0) return false;
     a.src = mk3(r0.x, r0.y, r0.z);
     h.scaling = r0.w;
     h.tau = r1.x;
@@ -379,6 +503,12 @@ __global__ void __launch_bounds__(kBlock) k_adj_rev(DevScene S, RenderArgs A) {
     const unsigned long long n_items =
         MODE == M_ADJSUB ? min(A.qcnt[Q_JOBS], A.job_cap) : min(A.qcnt[Q_SLOTS], A.slot_cap);
     unsigned long long *fetch = A.qcnt + (MODE == M_ADJSUB ? Q_WSUB : Q_WMAIN);
+    // fewer items than lanes are spread over the waves: a wave's step costs the
+    // union of its lanes' branches (a spline lane commits its tap sums every
+    // ten steps or so), so a few lanes step faster than 64
+    const unsigned long long waves = (unsigned long long)gridDim.x * (kBlock / 64);
+    const int share = (int)min(64ull, max(1ull, (n_items + waves - 1ull) / waves));
+    bool left = n_items > 0ull;  // items left (uniform)
     Var vsingle = var_from(S, A);
     Var &v = BATCH ? vars[threadIdx.x] : vsingle;
     int cur_cfg = -1;
@@ -410,17 +540,17 @@ __global__ void __launch_bounds__(kBlock) k_adj_rev(DevScene S, RenderArgs A) {
     Lane L{h, c, &v, S, A, cnt, &a, nullptr, nullptr, nullptr, true};
     const int lane = __lane_id();
     while (true) {
-        const unsigned long long need = __ballot(h.state == ST_NEED);
-        if (need) {
-            const int leader = __ffsll((long long)need) - 1;
-            unsigned long long base = 0;
-            if (lane == leader) base = atomicAdd(fetch, (unsigned long long)__popcll(need));
-            base = __shfl(base, leader);
-            if (h.state == ST_NEED) {
+        unsigned long long need = __ballot(h.state == ST_NEED);
+        if (need && left && share < 64) {
+            const int room = max(share - __popcll(__ballot(h.state != ST_NEED)), 0);
+            while (__popcll(need) > room) need &= need - 1ull;
+        }
+        if (need && left) {
+            const unsigned long long base = wave_take(fetch, need);
+            left = base + __popcll(need) < n_items;
+            if ((need >> lane) & 1ull) {
                 const unsigned long long idx = base + __popcll(need & ((1ull << lane) - 1ull));
-                if (idx >= n_items) {
-                    h.state = ST_DONE;
-                } else {
+                if (idx < n_items) {
                     if constexpr (BATCH) {
                         const int cfg = item_cfg<MODE>(A, idx);
                         if (cfg != cur_cfg) {
@@ -437,8 +567,10 @@ __global__ void __launch_bounds__(kBlock) k_adj_rev(DevScene S, RenderArgs A) {
             }
         }
         if (h.state == ST_REND) rev_end<FIELD, MODE>(L);
-        if (__ballot(h.state != ST_DONE) == 0ull) break;
-        if (__ballot(h.state == ST_RMARCH) == 0ull) continue;
+        if (__ballot(h.state == ST_RMARCH) == 0ull) {
+            if (__ballot(h.state != ST_NEED) == 0ull && !left) break;
+            continue;
+        }
         const FieldP F = v.f;
         bool r = h.state == ST_RMARCH;
         for (int k = 0; k < A.spc; ++k)

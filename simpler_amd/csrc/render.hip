@@ -61,7 +61,10 @@ constexpr int kBlock = 256;
 constexpr int kJtabLds = 128;  // Bessel table intervals staged in LDS (8 KiB)
 constexpr int kJtabLdsBatch = 1024;  // float4 (16 KiB): a batch's per-order tables in LDS
 constexpr int kMaxMode = 7;          // highest Bessel order (check_desc)
-constexpr int kJobVec = 4;           // float4 per entry of a next-event stack
+// float4 per entry of a next-event stack (the adjoint's re-trace adds one)
+__host__ __device__ constexpr int job_vec(int mode) { return mode == M_ADJDEF ? 5 : 4; }
+// modes whose next-event sub-paths go through the wave's stack
+__host__ __device__ constexpr bool stacked(int mode) { return mode == M_RENDER || mode == M_ADJDEF; }
 
 struct RenderArgs {
     float *image;
@@ -111,7 +114,7 @@ struct RenderArgs {
     // nee_skip; null: every next-event sub-path is traced
     const int *nee_cut;
     // next-event stacks of the render kernels (see nee_push): nq_cap entries
-    // of kJobVec float4 for each of the first nq_waves waves of the grid;
+    // of job_vec(mode) float4 for each of the first nq_waves waves of the grid;
     // wave_photons: photons a wave traces at a time (64 unless the launch has
     // fewer photons than lanes)
     float4 *nq;
@@ -1084,7 +1087,7 @@ __device__ __forceinline__ void wave_set(uint32_t *p, uint32_t v) {
 
 // nee_push: called by the lanes at a vertex (any subset of the wave); false
 // when the stack is full.
-template <int FIELD>
+template <int FIELD, int MODE>
 __device__ __forceinline__ bool nee_push(Lane &L) {
     const unsigned long long m = __ballot(1);
     const int lane = __lane_id(), leader = __ffsll((long long)m) - 1;
@@ -1094,12 +1097,13 @@ __device__ __forceinline__ bool nee_push(Lane &L) {
     if (i >= L.qcap) return false;
     const Hot &h = L.h;
     const Cold &c = L.c;
-    float4 *r = L.q + (size_t)i * kJobVec;
+    float4 *r = L.q + (size_t)i * job_vec(MODE);
     r[0] = make_float4(h.p.x, h.p.y, h.p.z, h.L);
     r[1] = make_float4(h.v.x, h.v.y, h.v.z, h.n0);
     r[2] = make_float4(h.g0.x, h.g0.y, h.g0.z, FIELD == kSources ? h.tau : h.scaling);
     r[3] = make_float4(__uint_as_float(c.pid_lo), __uint_as_float(c.pid_hi), __int_as_float(c.depth),
                        __int_as_float(L.cfg));
+    if constexpr (MODE == M_ADJDEF) adj_job_store(L, r + 4);
     // the wave's vector memory accesses are performed in order; this keeps
     // the compiler from moving the stores past a later entry's loads
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
@@ -1131,11 +1135,11 @@ __device__ __forceinline__ void nee_begin(Lane &L, f3 d, int phase) {
 }
 
 // Entry i of the wave's stack as the lane's sub-path.
-template <int FIELD, bool BATCH>
+template <int FIELD, int MODE, bool BATCH>
 __device__ __forceinline__ void nee_pop(Lane &L, uint32_t i) {
     Hot &h = L.h;
     Cold &c = L.c;
-    const float4 *r = L.q + (size_t)i * kJobVec;
+    const float4 *r = L.q + (size_t)i * job_vec(MODE);
     const float4 r0 = r[0], r1 = r[1], r2 = r[2], r3 = r[3];
     h.p = mk3(r0.x, r0.y, r0.z);
     h.pl = mk3(0.f, 0.f, 0.f);
@@ -1151,10 +1155,11 @@ __device__ __forceinline__ void nee_pop(Lane &L, uint32_t i) {
     c.pid_lo = __float_as_uint(r3.x);
     c.pid_hi = __float_as_uint(r3.y);
     c.depth = __float_as_int(r3.z);
-    if (BATCH) {
-        L.cfg = __float_as_int(r3.w);
+    if (BATCH) L.cfg = __float_as_int(r3.w);
+    if constexpr (MODE == M_ADJDEF)
+        adj_job_load(L, r[4]);
+    else if (BATCH)
         L.v = const_cast<Var *>(L.A.cfgs) + L.cfg;
-    }
     nee_begin(L, nee_dir(L), PH_JOB);
     start_segment(L, kLargeDist);
 }
@@ -1175,14 +1180,16 @@ __device__ __forceinline__ void vertex(Lane &L) {
     if (S.use_nee && !((double)(h.p.x - S.cam_o.x) < 1e-4)) {
         c.main_draw = c.draw;
         bool walk_on = false;  // no sub-path to trace here
-        if constexpr (MODE == M_RENDER) {
-            if (FIELD == kSpline && L.A.nee_fwd) {
+        if constexpr (stacked(MODE)) {
+            if (MODE == M_ADJDEF || (FIELD == kSpline && L.A.nee_fwd)) {
                 const f3 d = nee_dir(L);
                 walk_on = nee_skip(L, d);  // no splat
                 c.stream = 0;
                 c.draw = c.main_draw;
             }
-            walk_on = walk_on || nee_push<FIELD>(L);
+            if constexpr (MODE == M_ADJDEF)
+                if (!walk_on) adj_vertex_slot(L);
+            walk_on = walk_on || nee_push<FIELD, MODE>(L);
         }
         if (!walk_on) {
             c.mp = h.p;
@@ -1191,7 +1198,7 @@ __device__ __forceinline__ void vertex(Lane &L) {
             if (L.mc) *L.mc = make_float4(h.n0, h.g0.x, h.g0.y, h.g0.z);
             const f3 d = nee_dir(L);
             nee_begin(L, d, PH_NEE);
-            if (L.adj && nee_skip(L, d)) {  // no splat
+            if (!stacked(MODE) && L.adj && nee_skip(L, d)) {  // no splat
                 h.dead = true;
                 h.state = ST_SEG_END;
                 return;
@@ -1298,7 +1305,7 @@ __device__ __forceinline__ void nee_done(Lane &L, int res) {
             }
         }
     }
-    if (MODE == M_RENDER && c.phase == PH_JOB)
+    if (stacked(MODE) && c.phase == PH_JOB)
         h.state = ST_NEED;
     else
         nee_continue<FIELD>(L);
@@ -1482,6 +1489,48 @@ __device__ __forceinline__ void photon_init(Lane &L) {
     }
 }
 
+// Takes the next indices of a launch's work queue for the lanes of need, one
+// atomic per wave; returns the first one (uniform).
+__device__ __forceinline__ unsigned long long wave_take(unsigned long long *work, unsigned long long need) {
+    const int leader = __ffsll((long long)need) - 1;
+    unsigned long long base = 0;
+    if (__lane_id() == leader) base = atomicAdd(work, (unsigned long long)__popcll(need));
+    return (unsigned long long)(uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)base, leader) |
+           (unsigned long long)(uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(base >> 32), leader) << 32;
+}
+
+// The photon at index i over all configurations of a batch, and its
+// configuration c (the largest with prefix[c] <= i).
+__device__ __forceinline__ uint64_t batch_photon(const RenderArgs &A, unsigned long long i, int &c) {
+    int lo = 0, hi = A.n_cfg;
+    while (hi - lo > 1) {
+        const int mid = (lo + hi) >> 1;
+        if (A.prefix[mid] <= i)
+            lo = mid;
+        else
+            hi = mid;
+    }
+    c = lo;
+    return i - A.prefix[lo];
+}
+
+// A kernel argument at its offset of the argument segment, through a pointer
+// that the compiler takes for new at each call, so that what is read through
+// it is loaded where it is used and not kept in registers.  Read as plain
+// arguments, 150 scalars were spilled to vector registers and 45 vectors to
+// scratch in the m = 0 kernel (0 and 2 now), and the batched kernels fit three
+// waves per SIMD instead of four: 2^22 photons 447 -> 413 ms, the
+// 256-configuration sweep 391 -> 362 ms, 2^17 spline photons 172 -> 141 ms.
+template <class T>
+__device__ __forceinline__ const T &kernel_arg(size_t offset) {
+    using Segment = const __attribute__((address_space(4))) char *;
+    Segment p = (Segment)__builtin_amdgcn_kernarg_segment_ptr();
+    asm volatile("" : "+s"(p));
+    return *(const T *)(p + offset);
+}
+// the path kernels' arguments: a DevScene, then a RenderArgs
+constexpr size_t kArgsOffset = (sizeof(DevScene) + alignof(RenderArgs) - 1) / alignof(RenderArgs) * alignof(RenderArgs);
+
 }  // namespace simpler
 #include "adjoint_kernel.h"
 #include "prefilter.h"
@@ -1511,23 +1560,6 @@ namespace simpler {
 static_assert(5 * (sizeof(Cold) * kBlock + sizeof(uint32_t) * (C_N + kBlock / 64) + sizeof(float4) * (4 * kJtabLds + kBlock)) <=
                   160 * 1024,
               "five single-scene Bessel workgroups must fit one CU's LDS");
-
-// A kernel argument at its offset of the argument segment, through a pointer
-// that the compiler takes for new at each call, so that what is read through
-// it is loaded where it is used and not kept in registers.  Read as plain
-// arguments, 150 scalars were spilled to vector registers and 45 vectors to
-// scratch in the m = 0 kernel (0 and 2 now), and the batched kernels fit three
-// waves per SIMD instead of four: 2^22 photons 447 -> 413 ms, the
-// 256-configuration sweep 391 -> 362 ms, 2^17 spline photons 172 -> 141 ms.
-template <class T>
-__device__ __forceinline__ const T &kernel_arg(size_t offset) {
-    using Segment = const __attribute__((address_space(4))) char *;
-    Segment p = (Segment)__builtin_amdgcn_kernarg_segment_ptr();
-    asm volatile("" : "+s"(p));
-    return *(const T *)(p + offset);
-}
-// k_render's arguments: a DevScene, then a RenderArgs
-constexpr size_t kArgsOffset = (sizeof(DevScene) + alignof(RenderArgs) - 1) / alignof(RenderArgs) * alignof(RenderArgs);
 
 template <int FIELD, int MODE, bool BATCH, bool JLDS = false, int MM = -1, int GA = -1, int SPLAT = 0>
 __global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(FIELD == kBessel ? 5 : (FIELD == kSpline ? 2 : 1))))
@@ -1577,7 +1609,7 @@ k_render(DevScene S0, RenderArgs A0) {
             const int wave = __builtin_amdgcn_readfirstlane((int)((blockIdx.x * blockDim.x + tid) >> 6));
             L.qn = &nheld[tid >> 6];
             L.qcap = wave < A.nq_waves ? A.nq_cap : 0;
-            L.q = A.nq + (size_t)wave * A.nq_cap * kJobVec;
+            L.q = A.nq + (size_t)wave * A.nq_cap * job_vec(MODE);
             L.cfg = cfg;
         }
         // fetch: first the wave's next-event stack, then new photons, one
@@ -1591,7 +1623,7 @@ k_render(DevScene S0, RenderArgs A0) {
                 if (lane == 0) wave_set(L.qn, held - min(held, want));
                 __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
                 if (h.state == ST_NEED && rank < held) {
-                    nee_pop<FIELD, BATCH>(L, held - 1u - rank);
+                    nee_pop<FIELD, MODE, BATCH>(L, held - 1u - rank);
                 }
                 // lanes that found no entry take a photon
                 need = __ballot(h.state == ST_NEED && rank >= held);
@@ -1603,11 +1635,7 @@ k_render(DevScene S0, RenderArgs A0) {
             while (__popcll(need) > room) need &= need - 1ull;
         }
         if (need && left) {
-            const int leader = __ffsll((long long)need) - 1;
-            unsigned long long base = 0;
-            if (lane == leader) base = atomicAdd(A.work, (unsigned long long)__popcll(need));
-            base = (unsigned long long)(uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)base, leader) |
-                   (unsigned long long)(uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(base >> 32), leader) << 32;
+            const unsigned long long base = wave_take(A.work, need);
             left = base + __popcll(need) < A.n;
             if ((need >> lane) & 1ull) {
                 const unsigned long long rank = __popcll(need & ((1ull << lane) - 1ull));
@@ -1617,16 +1645,8 @@ k_render(DevScene S0, RenderArgs A0) {
                     if (BATCH) {
                         // index over all configurations (A.offset: the first
                         // photon of the launch's group of configurations)
-                        const unsigned long long gi = A.offset + idx;
-                        int lo = 0, hi = A.n_cfg;  // largest c with prefix[c] <= gi
-                        while (hi - lo > 1) {
-                            const int mid = (lo + hi) >> 1;
-                            if (A.prefix[mid] <= gi)
-                                lo = mid;
-                            else
-                                hi = mid;
-                        }
-                        pid = gi - A.prefix[lo];
+                        int lo;
+                        pid = batch_photon(A, A.offset + idx, lo);
                         L.v = const_cast<Var *>(A.cfgs + lo);  // its image pointer is set per launch
                         L.cfg = lo;
                     }
@@ -2258,13 +2278,17 @@ static int bessel_variant(const DevScene &S) {
 // the entries past a full stack, trace inline).
 constexpr int kStackEntries = 64, kStackWavesPerCU = 5 * kBlock / 64;
 
-// The launch's grid and the photons each wave traces at a time: a launch with
-// fewer photons than lanes spreads them over its waves, whose other lanes
-// take the next-event sub-paths.
+// The photons each wave of a launch of n traces at a time: a launch with fewer
+// photons than lanes spreads them over its waves, whose other lanes take the
+// next-event sub-paths.
+static int wave_share(uint64_t n, uint64_t waves) {
+    return (int)std::max<uint64_t>(1, std::min<uint64_t>(64, (n + waves - 1) / waves));
+}
+
+// A render's grid and wave_share.
 static void render_shape(const simpler_ctx *ctx, RenderArgs &A, int &blocks) {
     blocks = std::max(1, ctx->num_cu * ctx->bpc);
-    const uint64_t waves = (uint64_t)blocks * (uint64_t)(ctx->block / 64);
-    A.wave_photons = (int)std::max<uint64_t>(1, std::min<uint64_t>(64, (A.n + waves - 1) / waves));
+    A.wave_photons = wave_share(A.n, (uint64_t)blocks * (uint64_t)(ctx->block / 64));
 }
 
 template <int MODE>
@@ -2381,8 +2405,8 @@ int simpler_ctx_create(int device, simpler_ctx **out) {
     if (hipStreamCreateWithFlags(&ctx->own, hipStreamNonBlocking) != hipSuccess ||
         hipEventCreateWithFlags(&ctx->handoff, hipEventDisableTiming) != hipSuccess ||
         hipMalloc(&ctx->d_scratch, 16 * sizeof(unsigned long long)) != hipSuccess ||
-        hipMalloc(&ctx->d_nq, (size_t)(ctx->nq_waves = ctx->num_cu * kStackWavesPerCU) * kStackEntries * kJobVec *
-                                  sizeof(float4)) != hipSuccess) {
+        hipMalloc(&ctx->d_nq, (size_t)(ctx->nq_waves = ctx->num_cu * kStackWavesPerCU) * kStackEntries *
+                                  job_vec(M_RENDER) * sizeof(float4)) != hipSuccess) {
         (void)hipFree(ctx->d_scratch);
         if (ctx->handoff) (void)hipEventDestroy(ctx->handoff);
         if (ctx->own) (void)hipStreamDestroy(ctx->own);
@@ -2996,7 +3020,7 @@ static int render_impl(simpler_scene *sc, int64_t n_photons, int64_t n_total, ui
     if (!words) {
         words = ctx->d_scratch;
         stacks = ctx->d_nq;
-        stack_vec = (size_t)ctx->nq_waves * kStackEntries * kJobVec;
+        stack_vec = (size_t)ctx->nq_waves * kStackEntries * job_vec(M_RENDER);
     }
     int rc = scene_ready(sc);
     if (rc) return rc;
@@ -3029,7 +3053,7 @@ static int render_impl(simpler_scene *sc, int64_t n_photons, int64_t n_total, ui
     A.spc = ctx->spc;
     A.nq = stacks;
     A.nq_waves = ctx->nq_waves;
-    A.nq_cap = (int)std::min<size_t>(kStackEntries, stack_vec / ((size_t)ctx->nq_waves * kJobVec));
+    A.nq_cap = (int)std::min<size_t>(kStackEntries, stack_vec / ((size_t)ctx->nq_waves * job_vec(M_RENDER)));
     // zero work queue + counters (a fill kernel: safe under graph capture)
     hipLaunchKernelGGL(k_fill_u64, dim3(1), dim3(64), 0, ctx->cur, words, 16);
     if (!record && !accumulate) {
@@ -3377,12 +3401,24 @@ static int adjoint_deferred(simpler_ctx *ctx, dim3 grid, const DevScene &S, Rend
     const uint64_t off0 = A.offset;
     const dim3 tgrid(std::max(1, ctx->num_cu * def_trace_blocks(F)));
     const dim3 rgrid(std::max(1, ctx->num_cu * def_rev_blocks(F, BATCH)));
+    // the re-trace's next-event stacks: entries as many as the context's
+    // buffer holds for its waves
+    A.nq = ctx->d_nq;
+    A.nq_waves = (int)tgrid.x * (kBlock / 64);
+    A.nq_cap = (int)std::min<size_t>(kStackEntries, (size_t)ctx->nq_waves * kStackEntries * job_vec(M_RENDER) /
+                                                        ((size_t)A.nq_waves * job_vec(M_ADJDEF)));
+    // every photon with a next-event sub-path to trace stores its main path:
+    // a vertex per mean free path of the block and a few faces (more photons
+    // per chunk than their records fit would only be traced twice)
+    const double rec = 6.0 + 1.5 * (double)S.sigma_t * (double)(S.blockR.x - S.blockL.x);
+    const int64_t fit = std::max<int64_t>(kAdjChunkMin, (int64_t)(0.9 * (double)A.slotrec_cap / rec));
     const double caps[4] = {(double)A.job_cap, (double)A.jobrec_cap, (double)A.slot_cap, (double)A.slotrec_cap};
     int64_t start = 0;
     while (start < n) {
-        const int64_t m = std::min<int64_t>(ctx->adj_chunk, n - start);
+        const int64_t m = std::min<int64_t>(std::min<int64_t>(ctx->adj_chunk, fit), n - start);
         A.offset = off0 + (uint64_t)start;
         A.n = (uint64_t)m;
+        A.wave_photons = wave_share(A.n, (uint64_t)tgrid.x * (kBlock / 64));
         HIP_TRY(ctx, hipMemcpyAsync(ctx->d_q + 16, ctx->d_adj, 8 * sizeof(unsigned long long),
                                     hipMemcpyDeviceToDevice, ctx->cur));
         HIP_TRY(ctx, hipMemcpyAsync(ctx->d_q + 24, ctx->d_scratch + 8, 8 * sizeof(unsigned long long),
@@ -3391,7 +3427,7 @@ static int adjoint_deferred(simpler_ctx *ctx, dim3 grid, const DevScene &S, Rend
             HIP_TRY(ctx, hipMemcpyAsync(obj_backup, A.obj, n_obj * sizeof(double), hipMemcpyDeviceToDevice, ctx->cur));
         hipLaunchKernelGGL(k_fill_u64, dim3(1), dim3(64), 0, ctx->cur, ctx->d_scratch, 1);
         hipLaunchKernelGGL(k_fill_u64, dim3(1), dim3(64), 0, ctx->cur, ctx->d_q, Q_N);
-        hipLaunchKernelGGL((k_adjoint<F, M_ADJDEF, BATCH>), tgrid, dim3(kBlock), 0, ctx->cur, S, A);
+        hipLaunchKernelGGL((k_retrace<F, BATCH>), tgrid, dim3(kBlock), 0, ctx->cur, S, A);
         HIP_TRY(ctx, hipGetLastError());
         unsigned long long q[Q_OVER + 1];
         HIP_TRY(ctx, hipMemcpyAsync(q, ctx->d_q, sizeof(q), hipMemcpyDeviceToHost, ctx->cur));
