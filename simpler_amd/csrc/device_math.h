@@ -78,6 +78,18 @@ __device__ __forceinline__ float div10(float x) {
     return __builtin_fmaf(__builtin_fmaf(-q0, 10.0f, x), 0.1f, q0);
 }
 
+// The first active lane's x, as a scalar.
+__device__ __forceinline__ uint64_t uniform_u64(uint64_t x) {
+    return (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)x) |
+           (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(x >> 32)) << 32;
+}
+
+// a * b, never fused into an addition.
+__device__ __forceinline__ float mul_rn(float a, float b) {
+#pragma clang fp contract(off)
+    return a * b;
+}
+
 // Two-sum accumulation hi + lo += d (Kahan's compensated step).
 __device__ __forceinline__ void comp_add(float &hi, float &lo, float d) {
     const float y = d + lo;
