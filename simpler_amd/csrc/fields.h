@@ -47,6 +47,7 @@ struct DevScene {
     int precision;
     float egap, sgap;
     int n_src, n_coeff;
+    int src_lanes;  // kSplitSources: lanes that share one path, a power of two up to 64
     const float4 *src;  // (x, y, z, amplitude)
     const float *src_phase;
     float coeff_w[8];
@@ -65,7 +66,9 @@ struct DevScene {
     uint32_t seed_lo, seed_hi;
 };
 
-enum FieldKind { kBessel = 0, kSources = 1, kSpline = 2 };
+// kSplitSources: point sources of a path that S.src_lanes neighbouring lanes
+// trace together, each with a part of the sum.
+enum FieldKind { kBessel = 0, kSources = 1, kSpline = 2, kSplitSources = 3 };
 
 // Field parameters that differ between the configurations of a batched
 // launch (uniform in a single-scene launch, per lane in a batched one).
@@ -360,6 +363,55 @@ __device__ __forceinline__ void field_eval<kSources>(const DevScene &S, const Fi
         harmonics(AnyHarmonics{});
     n = S.n_o + acc;
     g = gacc;
+}
+
+// The sum of x over the `lanes` neighbouring lanes of a path, the same bits in
+// each of them (every turn adds two partners' values, in either order).
+__device__ __forceinline__ float lanes_sum(float x, int lanes) {
+    for (int k = 1; k < lanes; k <<= 1) x += __shfl_xor(x, k);
+    return x;
+}
+
+// field_eval<kSources> with the sources dealt out to the path's lanes, which
+// all come here together with the same arguments.
+template <>
+__device__ __forceinline__ void field_eval<kSplitSources>(const DevScene &S, const FieldP &F, f3 p, float, float tau,
+                                                          float &n, f3 &g) {
+    if (p.x > S.egap || p.x < S.sgap) {
+        n = S.n_o;
+        g = mk3(0.f, 0.f, 0.f);
+        return;
+    }
+    float acc = 0.f;
+    f3 gacc = mk3(0.f, 0.f, 0.f);
+    const float tshift = S.time_coupling * tau;
+    const int lanes = S.src_lanes;
+    const src4 *src = (const src4 *)F.src;
+    const auto harmonics = [&](auto one) {
+        const auto add = [&](src4 s, float phase) {
+            const SourceSums q = source_sums<decltype(one)::value>(S, F, p, s, phase - tshift);
+            acc += s.w * q.vs * q.ir;
+            const float common = -s.w * q.gs * q.ir * q.ir * q.ir;
+            gacc = gacc + common * q.dv;
+        };
+        int i = (int)__lane_id() & (lanes - 1);
+        for (; i + 3 * lanes < S.n_src; i += 4 * lanes) {
+            const src4 a = src[i], b = src[i + lanes], c = src[i + 2 * lanes], d = src[i + 3 * lanes];
+            const float pa = F.phase[i], pb = F.phase[i + lanes], pc = F.phase[i + 2 * lanes],
+                        pd = F.phase[i + 3 * lanes];
+            add(a, pa);
+            add(b, pb);
+            add(c, pc);
+            add(d, pd);
+        }
+        for (; i < S.n_src; i += lanes) add(src[i], F.phase[i]);
+    };
+    if (S.n_coeff == 1)
+        harmonics(OneHarmonic{});
+    else
+        harmonics(AnyHarmonics{});
+    n = S.n_o + lanes_sum(acc, lanes);
+    g = mk3(lanes_sum(gacc.x, lanes), lanes_sum(gacc.y, lanes), lanes_sum(gacc.z, lanes));
 }
 
 // Mirror-wrapped node index (spline.h:617-620, 636-644 for 1-D / 2-D; also

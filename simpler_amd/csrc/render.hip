@@ -1570,6 +1570,11 @@ k_render(DevScene S0, RenderArgs A0) {
     __shared__ float4 mcache[kBlock];
     __shared__ uint32_t nheld[kBlock / 64];  // entries of each wave's next-event stack
     constexpr bool STACK = MODE == M_RENDER;
+    // SPLIT: S.src_lanes neighbouring lanes trace each ray together, in the same
+    // control flow; one of them counts its events and writes its record
+    constexpr bool SPLIT = FIELD == kSplitSources;
+    static_assert(!SPLIT || MODE == M_RECORD, "only recorded rays are traced by several lanes");
+    __shared__ uint32_t uncounted[SPLIT ? C_N : 1];
     if (threadIdx.x < C_N) cnt[threadIdx.x] = 0u;
     if (STACK && (threadIdx.x & 63) == 0) nheld[threadIdx.x >> 6] = 0u;
     if (JLDS) {
@@ -1602,8 +1607,9 @@ k_render(DevScene S0, RenderArgs A0) {
         if (JLDS && !BATCH) vsingle.f.jtab = jlds;
         // batch: the lane's configuration, read from global memory (L1/L2
         // resident), replaced when the lane takes a photon of another one
-        Lane L{h, cold[tid], BATCH ? const_cast<Var *>(A.cfgs) + cfg : &vsingle, S, A, cnt, nullptr, &mcache[tid],
-               SPLAT ? &ps : nullptr, MODE == M_JVP ? &tan : nullptr};
+        const bool first = !SPLIT || (tid & (S.src_lanes - 1)) == 0;
+        Lane L{h, cold[tid], BATCH ? const_cast<Var *>(A.cfgs) + cfg : &vsingle, S, A, first ? cnt : uncounted, nullptr,
+               &mcache[tid], SPLAT ? &ps : nullptr, MODE == M_JVP ? &tan : nullptr};
         const int lane = __lane_id();
         if (STACK) {
             const int wave = __builtin_amdgcn_readfirstlane((int)((blockIdx.x * blockDim.x + tid) >> 6));
@@ -1635,10 +1641,13 @@ k_render(DevScene S0, RenderArgs A0) {
             while (__popcll(need) > room) need &= need - 1ull;
         }
         if (need && left) {
-            const unsigned long long base = wave_take(A.work, need);
-            left = base + __popcll(need) < A.n;
+            // the lanes that take: of a ray's lanes the first one
+            const unsigned long long take = SPLIT ? __ballot(h.state == ST_NEED && first) : need;
+            const unsigned long long base = wave_take(A.work, take);
+            left = base + __popcll(take) < A.n;
             if ((need >> lane) & 1ull) {
-                const unsigned long long rank = __popcll(need & ((1ull << lane) - 1ull));
+                const int taker = SPLIT ? lane & ~(S.src_lanes - 1) : lane;
+                const unsigned long long rank = __popcll(take & ((1ull << taker) - 1ull));
                 const unsigned long long idx = base + rank;
                 if (idx < A.n) {
                     uint64_t pid = A.offset + idx;
@@ -1686,6 +1695,7 @@ k_render(DevScene S0, RenderArgs A0) {
     }
     // counters: ER steps reduced over the wave, events from LDS, one atomic
     // per counter per wave / block
+    if (SPLIT) wave_steps /= (unsigned)S0.src_lanes;
     if (__lane_id() == 0 && wave_steps) atomicAdd(A0.counters + C_STEPS, wave_steps);
     __syncthreads();
     if (threadIdx.x < C_N && threadIdx.x != C_STEPS && cnt[threadIdx.x])
@@ -2291,6 +2301,19 @@ static void render_shape(const simpler_ctx *ctx, RenderArgs &A, int &blocks) {
     A.wave_photons = wave_share(A.n, (uint64_t)blocks * (uint64_t)(ctx->block / 64));
 }
 
+// The lanes that trace each recorded ray of a point-source field together: as
+// many as the launch has for it, with at least four sources each.  One lane
+// per ray leaves the chip to a few waves that each run the whole sum: 4,096 rays
+// of 10,200 sources 302 ms, with 64 lanes per ray 5.4 ms (now bound by the sum's
+// instructions); 65,536 rays 141 -> 76 ms with 4.  4,096 rays of 64 sources: 4.9
+// ms with one lane, 2.3 with 4, 2.0 with 16, 2.1 with 32; 262,144 rays, which
+// fill the lanes by themselves: 13.3 ms with one, 16.7 with 2.
+static int source_lanes(uint64_t rays, int n_src, uint64_t lanes) {
+    int k = 1;
+    while (k < 64 && n_src >= 8 * k && rays * 2 * k <= lanes) k *= 2;
+    return k;
+}
+
 template <int MODE>
 static void launch_render(simpler_ctx *ctx, int field, const DevScene &S, RenderArgs A) {
     int blocks = 0;
@@ -2322,7 +2345,17 @@ static void launch_render(simpler_ctx *ctx, int field, const DevScene &S, Render
             else
                 hipLaunchKernelGGL((k_render<kBessel, MODE, false>), grid, block, 0, ctx->cur, S, A);
             break;
-        case SIMPLER_FIELD_SOURCES: hipLaunchKernelGGL((k_render<kSources, MODE, false>), grid, block, 0, ctx->cur, S, A); break;
+        case SIMPLER_FIELD_SOURCES:
+            if constexpr (MODE == M_RECORD) {
+                DevScene T = S;
+                T.src_lanes = source_lanes(A.n, S.n_src, (uint64_t)blocks * (uint64_t)ctx->block);
+                if (T.src_lanes > 1) {
+                    hipLaunchKernelGGL((k_render<kSplitSources, M_RECORD, false>), grid, block, 0, ctx->cur, T, A);
+                    break;
+                }
+            }
+            hipLaunchKernelGGL((k_render<kSources, MODE, false>), grid, block, 0, ctx->cur, S, A);
+            break;
         default: hipLaunchKernelGGL((k_render<kSpline, MODE, false>), grid, block, 0, ctx->cur, S, A); break;
     }
 }
