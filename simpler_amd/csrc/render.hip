@@ -1971,6 +1971,7 @@ struct simpler_ctx {
     int nq_waves = 0;
     int num_cu = 256;
     int block = 256, spc = 32, bpc = 4;
+    bool shape_set = false;  // chosen by the caller or the autotuner: renders take it as it is
     int splat = 0;  // splat strategy: 0 per-lane atomics, 1 wave-aggregated
     int live = 0;  // scenes and batches not yet destroyed
     float *d_log = nullptr;  // adjoint segment logs (grown on demand)
@@ -2295,9 +2296,30 @@ static int wave_share(uint64_t n, uint64_t waves) {
     return (int)std::max<uint64_t>(1, std::min<uint64_t>(64, (n + waves - 1) / waves));
 }
 
-// A render's grid and wave_share.
-static void render_shape(const simpler_ctx *ctx, RenderArgs &A, int &blocks) {
-    blocks = std::max(1, ctx->num_cu * ctx->bpc);
+// A render's grid, march steps per event phase and wave_share.  Where the
+// caller (or the autotuner) has chosen a launch shape it is taken as it is.
+// Otherwise a launch takes as many workgroups of 256 as give each wave eight
+// photons, within [lo, hi] per CU: a wave with a few photons issues nearly as
+// many instructions per step as a full one, so more waves than that only slow
+// the longest photon's down, and fewer leave SIMDs idle.  hi is what the kernel
+// keeps resident (five for single Bessel scenes, four for their batches, two
+// for the spline's 256 registers), and two for point sources, whose long step
+// two waves per SIMD fill.  A Bessel launch with many photons for every lane
+// also takes 128 steps per event phase.  Measured, the fixed four workgroups
+// per CU and 32 steps -> this rule: 16,384 Bessel photons 13.4 -> 11.0 ms, 2^22
+// photons 414 -> 364 ms, 4,096 spline photons 40.8 -> 31.4 ms, 2^17 142 -> 136 ms,
+// 4,096 photons of 16 sources 111 -> 55 ms, 2^15 135 -> 119 ms, 2^17 242 -> 216 ms.
+static void render_shape(const simpler_ctx *ctx, RenderArgs &A, int &blocks, int field, bool batch) {
+    if (ctx->shape_set) {
+        blocks = std::max(1, ctx->num_cu * ctx->bpc);
+    } else {
+        const bool bessel = field == SIMPLER_FIELD_BESSEL;
+        const uint64_t cus = (uint64_t)std::max(1, ctx->num_cu);
+        const uint64_t lo = bessel ? 2 : 1, hi = bessel ? (batch ? 4 : 5) : 2;
+        const uint64_t want = (A.n + 31) / 32;  // four waves of eight photons
+        blocks = (int)std::min(hi * cus, std::max(lo * cus, want));
+        if (bessel && !batch && A.n >= 4 * 256 * hi * cus) A.spc = std::max(A.spc, 128);
+    }
     A.wave_photons = wave_share(A.n, (uint64_t)blocks * (uint64_t)(ctx->block / 64));
 }
 
@@ -2316,8 +2338,8 @@ static int source_lanes(uint64_t rays, int n_src, uint64_t lanes) {
 
 template <int MODE>
 static void launch_render(simpler_ctx *ctx, int field, const DevScene &S, RenderArgs A) {
-    int blocks = 0;
-    render_shape(ctx, A, blocks);
+    int blocks = std::max(1, ctx->num_cu * ctx->bpc);
+    if (MODE == M_RENDER) render_shape(ctx, A, blocks, field, false);
     const dim3 grid(blocks), block(ctx->block);
     switch (field) {
         case SIMPLER_FIELD_BESSEL:
@@ -2517,6 +2539,7 @@ int simpler_ctx_set_tuning(simpler_ctx *ctx, int block_size, int steps_per_chunk
         if (blocks_per_cu < 1 || blocks_per_cu > 64) return fail(ctx, SIMPLER_ERR_INVALID, "blocks_per_cu out of range [1,64]");
         ctx->bpc = blocks_per_cu;
     }
+    ctx->shape_set |= block_size || steps_per_chunk || blocks_per_cu;
     return SIMPLER_OK;
 }
 
@@ -2551,6 +2574,8 @@ int simpler_autotune(simpler_scene *sc, int64_t n_photons, int X, int Y, int Z, 
     float best_ms = INFINITY;
     rc = SIMPLER_OK;
     bool warm = false;
+    const bool was_set = ctx->shape_set;
+    ctx->shape_set = true;
     // launch shapes with per-lane splats, then the aggregated splat at the
     // best shape (the strategy changes the event phase, not the march)
     for (int stage = 0; stage < (has_agg ? 2 : 1); ++stage)
@@ -2589,6 +2614,7 @@ int simpler_autotune(simpler_scene *sc, int64_t n_photons, int X, int Y, int Z, 
     ctx->spc = best[1];
     ctx->bpc = best[2];
     ctx->splat = best[3];
+    ctx->shape_set = was_set || best_ms < INFINITY;
     (void)hipEventDestroy(e0);
     (void)hipEventDestroy(e1);
     (void)hipFree(img);
@@ -3743,7 +3769,7 @@ static int batch_launch(simpler_batch *b, float *images, int accumulate, hipStre
     }
     if (b->total > 0) {
         int blocks = 0;
-        render_shape(ctx, A, blocks);
+        render_shape(ctx, A, blocks, b->field, true);
         if (b->field == SIMPLER_FIELD_SOURCES)
             hipLaunchKernelGGL((k_render<kSources, M_RENDER, true>), dim3(blocks), dim3(ctx->block), 0, stream, b->S,
                                A);
@@ -3754,7 +3780,7 @@ static int batch_launch(simpler_batch *b, float *images, int accumulate, hipStre
                 if (k) hipLaunchKernelGGL(k_fill_u64, dim3(1), dim3(64), 0, stream, ctx->d_scratch, 1);
                 A.offset = b->g_start[k];
                 A.n = b->g_count[k];
-                render_shape(ctx, A, blocks);
+                render_shape(ctx, A, blocks, b->field, true);
                 const dim3 grid(blocks), block(ctx->block);
                 switch (b->g_mode[k]) {
                     case 0: batch_bessel_launch<0>(grid, block, stream, b->S, A); break;
