@@ -29,7 +29,8 @@ HIP_FLAGS = [
 ]
 
 HIP_SOURCES = ["render.hip"]
-HIP_DEPS = ["render.hip", "fields.h", "device_math.h", "adjoint.h", "adjoint_kernel.h", "prefilter.h"]
+HIP_DEPS = ["render.hip", "fields.h", "device_math.h", "adjoint.h", "adjoint_kernel.h", "prefilter.h",
+            "render_loop.inl"]
 
 
 def _run(cmd):

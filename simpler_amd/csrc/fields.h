@@ -137,7 +137,7 @@ __device__ __forceinline__ void bessel_eval(const DevScene &S, const FieldP &F, 
     float r2;
     if (GA == 2) {
         rho = mk3(p.x - S.pu.x, p.y - S.pu.y, 0.f);
-        r2 = rho.x * rho.x + rho.y * rho.y;
+        r2 = __builtin_fmaf(rho.x, rho.x, rho.y * rho.y);  // fused by hand, as dot
     } else {
         const f3 q = p - S.pu;
         const float t = dot(q, S.uz);
@@ -212,7 +212,7 @@ template <int GA>
 __device__ __forceinline__ void bessel_rho(const DevScene &S, f3 p, f3 &rho, float &r2) {
     if (GA == 2) {
         rho = mk3(p.x - S.pu.x, p.y - S.pu.y, 0.f);
-        r2 = rho.x * rho.x + rho.y * rho.y;
+        r2 = __builtin_fmaf(rho.x, rho.x, rho.y * rho.y);  // fused by hand, as dot
     } else {
         const f3 q = p - S.pu;
         const float t = dot(q, S.uz);
