@@ -360,7 +360,7 @@ __device__ __forceinline__ void adj_log_sub(Lane &L, f3 nrm) {
 // Deferred image adjoint.  The re-trace (M_ADJDEF) does not run backward
 // runs itself: a splat that touches G queues a sub-path job (its end state,
 // step pattern, face records, adjoint seeds and start point), and a photon
-// with a queued next-event sub-path stores its main-path log in a slot when
+// with a traced next-event sub-path stores its main-path log in a slot when
 // it ends.  k_adj_rev then runs the jobs (M_ADJSUB: each adds its vertex
 // adjoint to the slot's record) and afterwards the slots (M_ADJMAIN), every
 // lane of a wave running backwards, instead of the few reversing lanes of a
