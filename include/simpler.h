@@ -277,7 +277,11 @@ int simpler_render_host_noalloc(simpler_scene *scene, int64_t n_photons,
  * exit direction inside the medium, out_len = optical path length at the exit
  * point, out_status = 1 reached the sensor face, 0 lost through another face,
  * -1 LargeDist exhausted, -2 abandoned (2^20 face events), -4 rejected by
- * the emitter lens.
+ * the emitter lens.  A ray's outputs do not depend on the other rays of the
+ * call or on the launch shape.  The sum over more than 16 point sources is
+ * taken in partial sums whose number follows from the number of sources; the
+ * renders and simpler_jvp_rays add the sources one after another (they differ
+ * from it by the rounding of the sum).
  */
 int simpler_trace_rays(simpler_scene *scene, int64_t n_rays, uint64_t seed,
                        uint64_t photon_offset, float *out_pos_dev,

@@ -47,7 +47,7 @@ struct DevScene {
     int precision;
     float egap, sgap;
     int n_src, n_coeff;
-    int src_lanes;  // kSplitSources: lanes that share one path, a power of two up to 64
+    int src_lanes, src_parts;  // kSplitSources ..: lanes that share one path, partial sums of its source sum
     const float4 *src;  // (x, y, z, amplitude)
     const float *src_phase;
     float coeff_w[8];
@@ -66,9 +66,10 @@ struct DevScene {
     uint32_t seed_lo, seed_hi;
 };
 
-// kSplitSources: point sources of a path that S.src_lanes neighbouring lanes
-// trace together, each with a part of the sum.
-enum FieldKind { kBessel = 0, kSources = 1, kSpline = 2, kSplitSources = 3 };
+// kSplitSources ..: point sources of a path that S.src_lanes neighbouring lanes
+// trace together, each with a part of the sum (source_parts): kSplitSources + j
+// with 2^j partial sums per lane, kSerialSources with all of them in one.
+enum FieldKind { kBessel = 0, kSources = 1, kSpline = 2, kSplitSources = 3, kSerialSources = 7 };
 
 // Field parameters that differ between the configurations of a batched
 // launch (uniform in a single-scene launch, per lane in a batched one).
@@ -365,54 +366,176 @@ __device__ __forceinline__ void field_eval<kSources>(const DevScene &S, const Fi
     g = gacc;
 }
 
+// The value and gradient sums of some point sources; add: one source's terms,
+// rounded as in field_eval<kSources>.
+struct SourceAcc {
+    float v = 0.f;
+    f3 g = mk3(0.f, 0.f, 0.f);
+    __device__ __forceinline__ void add(const SourceSums &q, float amp) {
+        v = __builtin_fmaf(amp * q.vs, q.ir, v);
+        const float common = -amp * q.gs * q.ir * q.ir * q.ir;
+        g = fma3(common, q.dv, g);
+    }
+};
+__device__ __forceinline__ SourceAcc operator+(const SourceAcc &a, const SourceAcc &b) {
+    SourceAcc c;
+    c.v = a.v + b.v;
+    c.g = a.g + b.g;
+    return c;
+}
+
+// The partial sums P (a power of two) of a recorded ray's source sum: partial r
+// adds the sources r, r + P, r + 2P, .. in order, and the partials are combined
+// in a tree, r with r ^ P/2 first, r with r ^ 1 last.  P follows from the number of
+// sources alone, so that a ray has the same bits in every launch, whichever
+// lanes hold its partials (source_lanes): as many as leave four sources to each
+// and fit one wave.  Up to 16 sources, the counts that the adjoint takes, P is 1,
+// the sum of the other kernels; several lanes per ray would gain little there
+// (4,096 rays of 16 sources 1.5 ms with one lane, 1.4 with four).
+__host__ __device__ constexpr int source_parts(int n_src) {
+    return n_src <= 16 ? 1 : (n_src < 32 ? 4 : (n_src < 64 ? 8 : (n_src < 128 ? 16 : (n_src < 256 ? 32 : 64))));
+}
+
 // The sum of x over the `lanes` neighbouring lanes of a path, the same bits in
 // each of them (every turn adds two partners' values, in either order).
 __device__ __forceinline__ float lanes_sum(float x, int lanes) {
-    for (int k = 1; k < lanes; k <<= 1) x += __shfl_xor(x, k);
+    for (int k = lanes >> 1; k > 0; k >>= 1) x += __shfl_xor(x, k);
     return x;
 }
 
-// field_eval<kSources> with the sources dealt out to the path's lanes, which
-// all come here together with the same arguments.
-template <>
-__device__ __forceinline__ void field_eval<kSplitSources>(const DevScene &S, const FieldP &F, f3 p, float, float tau,
-                                                          float &n, f3 &g) {
+// Partials first, first + stride, .. (W of them, W * stride = P), combined; four
+// sources' loads are in flight together.
+template <int W, class P4, class P1, class Term>
+__device__ __forceinline__ SourceAcc lane_partials(int n, int first, int stride, P4 src, P1 phase, Term &&term) {
+    constexpr int U = W < 4 ? 4 : W;  // sources per turn
+    SourceAcc a[W];
+    int i = first;
+    for (; i + (U - 1) * stride < n; i += U * stride) {
+#pragma unroll
+        for (int r = 0; r < U; r += 4) {
+            const int j = i + r * stride;
+            const src4 s0 = src[j], s1 = src[j + stride], s2 = src[j + 2 * stride], s3 = src[j + 3 * stride];
+            const float p0 = phase[j], p1 = phase[j + stride], p2 = phase[j + 2 * stride], p3 = phase[j + 3 * stride];
+            a[r % W].add(term(s0, p0), s0.w);
+            a[(r + 1) % W].add(term(s1, p1), s1.w);
+            a[(r + 2) % W].add(term(s2, p2), s2.w);
+            a[(r + 3) % W].add(term(s3, p3), s3.w);
+        }
+    }
+    if constexpr (W == 1) {
+        for (; i < n; i += stride) {
+            const src4 s = src[i];
+            a[0].add(term(s, phase[i]), s.w);
+        }
+    } else {
+#pragma unroll
+        for (int r = 0; r < U - 1; ++r) {
+            if (i + r * stride < n) {
+                const src4 s = src[i + r * stride];
+                a[r % W].add(term(s, phase[i + r * stride]), s.w);
+            }
+        }
+    }
+#pragma unroll
+    for (int h = W / 2; h > 0; h /= 2)
+#pragma unroll
+        for (int r = 0; r < h; ++r) a[r] = a[r] + a[r + h];
+    return a[0];
+}
+
+// All P >= 4 partials in one lane, four at a time in the order in which the
+// tree takes them.
+template <class P4, class P1, class Term>
+__device__ __forceinline__ SourceAcc serial_partials(int n, int parts, P4 src, P1 phase, Term &&term) {
+    const int fours = parts / 4;
+    SourceAcc s0, s1, s2, s3, v;
+#pragma unroll 1
+    for (int q = 0; q < fours; ++q) {
+        // the reversed bits of q: quads q, q + 1 (q even) are fours / 2 apart
+        const int first = (int)(__brev((uint32_t)q) >> 28) * fours >> 4;
+        SourceAcc a, b, c, d;
+        int i = first;
+#pragma unroll 1
+        for (; i + 3 * fours < n; i += parts) {
+            const src4 sa = src[i], sb = src[i + fours], sc = src[i + 2 * fours], sd = src[i + 3 * fours];
+            const float pa = phase[i], pb = phase[i + fours], pc = phase[i + 2 * fours], pd = phase[i + 3 * fours];
+            a.add(term(sa, pa), sa.w);
+            b.add(term(sb, pb), sb.w);
+            c.add(term(sc, pc), sc.w);
+            d.add(term(sd, pd), sd.w);
+        }
+        if (i < n) a.add(term(src[i], phase[i]), src[i].w);
+        if (i + fours < n) b.add(term(src[i + fours], phase[i + fours]), src[i + fours].w);
+        if (i + 2 * fours < n) c.add(term(src[i + 2 * fours], phase[i + 2 * fours]), src[i + 2 * fours].w);
+        v = (a + c) + (b + d);
+        if (q & 1) {
+            v = s0 + v;
+            if (q & 2) {
+                v = s1 + v;
+                if (q & 4) {
+                    v = s2 + v;
+                    if (q & 8)
+                        v = s3 + v;
+                    else
+                        s3 = v;
+                } else {
+                    s2 = v;
+                }
+            } else {
+                s1 = v;
+            }
+        } else {
+            s0 = v;
+        }
+    }
+    return v;
+}
+
+// field_eval<kSources> with the partial sums dealt out to the path's lanes, which
+// all come here together with the same arguments: W per lane, all in one lane
+// if W is 0 (through scalar loads, as for_sources).
+template <int W>
+__device__ __forceinline__ void sources_shared(const DevScene &S, const FieldP &F, f3 p, float tau, float &n, f3 &g) {
     if (p.x > S.egap || p.x < S.sgap) {
         n = S.n_o;
         g = mk3(0.f, 0.f, 0.f);
         return;
     }
-    float acc = 0.f;
-    f3 gacc = mk3(0.f, 0.f, 0.f);
-    const float tshift = S.time_coupling * tau;
+    SourceAcc sum;
+    const float tshift = mul_rn(S.time_coupling, tau);
     const int lanes = S.src_lanes;
-    const src4 *src = (const src4 *)F.src;
     const auto harmonics = [&](auto one) {
-        const auto add = [&](src4 s, float phase) {
-            const SourceSums q = source_sums<decltype(one)::value>(S, F, p, s, phase - tshift);
-            acc += s.w * q.vs * q.ir;
-            const float common = -s.w * q.gs * q.ir * q.ir * q.ir;
-            gacc = gacc + common * q.dv;
+        const auto term = [&](src4 s, float phase) {
+            return source_sums<decltype(one)::value>(S, F, p, s, phase - tshift);
         };
-        int i = (int)__lane_id() & (lanes - 1);
-        for (; i + 3 * lanes < S.n_src; i += 4 * lanes) {
-            const src4 a = src[i], b = src[i + lanes], c = src[i + 2 * lanes], d = src[i + 3 * lanes];
-            const float pa = F.phase[i], pb = F.phase[i + lanes], pc = F.phase[i + 2 * lanes],
-                        pd = F.phase[i + 3 * lanes];
-            add(a, pa);
-            add(b, pb);
-            add(c, pc);
-            add(d, pd);
+        if constexpr (W == 0) {
+            typedef const __attribute__((address_space(4))) src4 *Uniform4;
+            typedef const __attribute__((address_space(4))) float *Uniform1;
+            sum = serial_partials(S.n_src, S.src_parts, (Uniform4)uniform_u64((uint64_t)F.src),
+                                  (Uniform1)uniform_u64((uint64_t)F.phase), term);
+        } else {
+            sum = lane_partials<W>(S.n_src, (int)__lane_id() & (lanes - 1), lanes, (const src4 *)F.src, F.phase, term);
         }
-        for (; i < S.n_src; i += lanes) add(src[i], F.phase[i]);
     };
     if (S.n_coeff == 1)
         harmonics(OneHarmonic{});
     else
         harmonics(AnyHarmonics{});
-    n = S.n_o + lanes_sum(acc, lanes);
-    g = mk3(lanes_sum(gacc.x, lanes), lanes_sum(gacc.y, lanes), lanes_sum(gacc.z, lanes));
+    n = S.n_o + (W ? lanes_sum(sum.v, lanes) : sum.v);
+    g = W ? mk3(lanes_sum(sum.g.x, lanes), lanes_sum(sum.g.y, lanes), lanes_sum(sum.g.z, lanes)) : sum.g;
 }
+#define SIMPLER_SOURCES(K, W)                                                                                          \
+    template <>                                                                                                        \
+    __device__ __forceinline__ void field_eval<K>(const DevScene &S, const FieldP &F, f3 p, float, float tau,          \
+                                                  float &n, f3 &g) {                                                   \
+        sources_shared<W>(S, F, p, tau, n, g);                                                                         \
+    }
+SIMPLER_SOURCES(kSplitSources, 1)
+SIMPLER_SOURCES(kSplitSources + 1, 2)
+SIMPLER_SOURCES(kSplitSources + 2, 4)
+SIMPLER_SOURCES(kSplitSources + 3, 8)
+SIMPLER_SOURCES(kSerialSources, 0)
+#undef SIMPLER_SOURCES
 
 // Mirror-wrapped node index (spline.h:617-620, 636-644 for 1-D / 2-D; also
 // applied in 3-D).  One reflection covers i in [-(n-1), 2n-2], i.e. every

@@ -1568,14 +1568,14 @@ static_assert(5 * (sizeof(Cold) * kBlock + sizeof(uint32_t) * (C_N + kBlock / 64
               "five single-scene Bessel workgroups must fit one CU's LDS");
 
 template <int FIELD, int MODE, bool BATCH, bool JLDS = false, int MM = -1, int GA = -1, int SPLAT = 0>
-__global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(FIELD == kBessel ? 5 : (FIELD == kSpline ? 2 : 1))))
+__global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(FIELD == kBessel ? 5 : (FIELD == kSpline ? 2 : (FIELD > kSplitSources ? 4 : 1)))))
 k_render(DevScene S0, RenderArgs A0) {
     __shared__ Cold cold[kBlock];
     __shared__ uint32_t cnt[C_N];
     __shared__ float4 jlds[JLDS ? (BATCH ? kJtabLdsBatch : 4 * kJtabLds) : 1];
     __shared__ float4 mcache[kBlock];
     __shared__ uint32_t nheld[kBlock / 64];  // entries of each wave's next-event stack
-    constexpr bool STACK = MODE == M_RENDER, SPLIT = FIELD == kSplitSources;
+    constexpr bool STACK = MODE == M_RENDER, SPLIT = FIELD >= kSplitSources;
     __shared__ uint32_t uncounted[SPLIT ? C_N : 1];
     if (threadIdx.x < C_N) cnt[threadIdx.x] = 0u;
     if (STACK && (threadIdx.x & 63) == 0) nheld[threadIdx.x >> 6] = 0u;
@@ -2266,17 +2266,39 @@ static void render_shape(const simpler_ctx *ctx, RenderArgs &A, int &blocks, int
     A.wave_photons = wave_share(A.n, (uint64_t)blocks * (uint64_t)(ctx->block / 64));
 }
 
-// The lanes that trace each recorded ray of a point-source field together: as
-// many as the launch has for it, with at least four sources each.  One lane
-// per ray leaves the chip to a few waves that each run the whole sum: 4,096 rays
-// of 10,200 sources 302 ms, with 64 lanes per ray 5.4 ms (now bound by the sum's
-// instructions); 65,536 rays 141 -> 76 ms with 4.  4,096 rays of 64 sources: 4.9
-// ms with one lane, 2.3 with 4, 2.0 with 16, 2.1 with 32; 262,144 rays, which
-// fill the lanes by themselves: 13.3 ms with one, 16.7 with 2.
-static int source_lanes(uint64_t rays, int n_src, uint64_t lanes) {
-    int k = 1;
-    while (k < 64 && n_src >= 8 * k && rays * 2 * k <= lanes) k *= 2;
+// The lanes that trace each recorded ray of a point-source field together: one
+// where the rays fill the launch by themselves, else as many as it has for them,
+// with one to eight of the sum's partials each.  One lane per ray leaves the
+// chip to a few waves that each run the whole sum, and its latency: with one
+// lane -> this rule 4,096 rays of 10,200 sources 129 -> 5.3 ms (bound by the
+// sum's instructions), 65,536 rays 170 -> 74 ms, 4,096 rays of 64 sources 1.27
+// -> 0.46 ms, 65,536 rays of 300 sources 7.0 -> 4.1 ms.  Where the rays fill the
+// lanes, one lane per ray saves the step around the sum: 262,144 rays of 64
+// sources 2.9 ms, with 16 lanes each 6.4.  More than eight partials in one lane
+// take its registers; fewer lanes than an eighth of the partials are not used.
+static int source_lanes(uint64_t rays, int parts, uint64_t lanes) {
+    if (rays >= lanes) return 1;
+    int k = parts;
+    while (k > 1 && 8 * k > parts && rays * k > lanes) k /= 2;
     return k;
+}
+
+static void launch_shared_sources(simpler_ctx *ctx, dim3 grid, dim3 block, DevScene S, const RenderArgs &A) {
+    S.src_parts = source_parts(S.n_src);
+    S.src_lanes = source_lanes(A.n, S.src_parts, (uint64_t)grid.x * block.x);
+#define SIMPLER_RAYS(K) hipLaunchKernelGGL((k_render<K, M_RECORD, false>), grid, block, 0, ctx->cur, S, A)
+    if (S.src_parts == 1)
+        SIMPLER_RAYS(kSources);
+    else if (S.src_lanes == 1)
+        SIMPLER_RAYS(kSerialSources);
+    else
+        switch (S.src_parts / S.src_lanes) {
+            case 1: SIMPLER_RAYS(kSplitSources); break;
+            case 2: SIMPLER_RAYS(kSplitSources + 1); break;
+            case 4: SIMPLER_RAYS(kSplitSources + 2); break;
+            default: SIMPLER_RAYS(kSplitSources + 3); break;
+        }
+#undef SIMPLER_RAYS
 }
 
 template <int MODE>
@@ -2311,15 +2333,10 @@ static void launch_render(simpler_ctx *ctx, int field, const DevScene &S, Render
                 hipLaunchKernelGGL((k_render<kBessel, MODE, false>), grid, block, 0, ctx->cur, S, A);
             break;
         case SIMPLER_FIELD_SOURCES:
-            if constexpr (MODE == M_RECORD) {
-                DevScene T = S;
-                T.src_lanes = source_lanes(A.n, S.n_src, (uint64_t)blocks * (uint64_t)ctx->block);
-                if (T.src_lanes > 1) {
-                    hipLaunchKernelGGL((k_render<kSplitSources, M_RECORD, false>), grid, block, 0, ctx->cur, T, A);
-                    break;
-                }
-            }
-            hipLaunchKernelGGL((k_render<kSources, MODE, false>), grid, block, 0, ctx->cur, S, A);
+            if constexpr (MODE == M_RECORD)
+                launch_shared_sources(ctx, grid, block, S, A);
+            else
+                hipLaunchKernelGGL((k_render<kSources, MODE, false>), grid, block, 0, ctx->cur, S, A);
             break;
         default: hipLaunchKernelGGL((k_render<kSpline, MODE, false>), grid, block, 0, ctx->cur, S, A); break;
     }
