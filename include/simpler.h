@@ -480,18 +480,17 @@ int simpler_ctx_get_splat(simpler_ctx *ctx, int *strategy);
  * that splats into the objective runs the sub-path backwards at once, and the
  * photon's main path when it ends, while the other lanes of its wave march
  * on; 1 (default) = deferred: the re-trace queues each such sub-path (its log
- * and adjoint seed) and the main-path log of each photon with a next-event
- * sub-path, then a second kernel runs the queued sub-paths and a third the main
- * paths, every lane reversing.
+ * and adjoint seed) and the main-path log of each photon with one (of the last
+ * photons of a chunk: with any next-event sub-path), then a second kernel runs
+ * the queued sub-paths and a third the main paths, every lane reversing.
  * queue_capacity c (0 keeps the current value, default 2^23; else
  * 64 <= c <= 2^26) sizes the queues of one chunk of photons: c sub-paths
  * with c sub-path records, c main paths with 8 c main-path records, 768 c
  * bytes of device memory (6 GiB at the default), allocated on first use and
- * kept by the context.  The chunk starts at 2^22 photons (less where the mean
- * path's main-path records would pass 90 % of their queue), halves when a
+ * kept by the context.  The chunk starts at 2^22 photons, halves when a
  * chunk's queues overflow (the chunk is then traced again) and doubles, up
- * to 2^24, after a chunk that filled no queue past 40 %; at 2^14 photons an
- * overflowing chunk runs inline.  Both schedules give the same objective
+ * to 2^24, after a chunk that left room for twice its photons; when a chunk of
+ * 2^14 photons overflows the rest of the call runs inline.  Both schedules give the same objective
  * and counts, and the same gradient up to the order of float additions. */
 int simpler_ctx_set_adjoint_schedule(simpler_ctx *ctx, int schedule, int64_t queue_capacity);
 int simpler_ctx_get_adjoint_schedule(simpler_ctx *ctx, int *schedule, int64_t *queue_capacity);

@@ -60,6 +60,7 @@ struct AdjState {
     // whether that main path's log was full
     int jslot, jvert;
     bool jtrunc;
+    bool push;      // deferred re-trace: the photon's sub-paths may go to the wave's stack
     int cfg;        // batched kernels: the lane's configuration
     bool pending, trunc_main, trunc_sub;
     double F;
@@ -360,12 +361,12 @@ __device__ __forceinline__ void adj_log_sub(Lane &L, f3 nrm) {
 // Deferred image adjoint.  The re-trace (M_ADJDEF) does not run backward
 // runs itself: a splat that touches G queues a sub-path job (its end state,
 // step pattern, face records, adjoint seeds and start point), and a photon
-// with a traced next-event sub-path stores its main-path log in a slot when
-// it ends.  k_adj_rev then runs the jobs (M_ADJSUB: each adds its vertex
-// adjoint to the slot's record) and afterwards the slots (M_ADJMAIN), every
-// lane of a wave running backwards, instead of the few reversing lanes of a
-// mostly marching wave.  A queue that fills sets qcnt[Q_OVER]; the host then
-// re-runs that chunk of photons in smaller pieces.
+// with a sub-path that did, or that was left on the wave's stack, stores its
+// main-path log in a slot when it ends.  k_adj_rev then runs the jobs (M_ADJSUB:
+// each adds its vertex adjoint to the slot's record) and afterwards the slots
+// (M_ADJMAIN), every lane of a wave running backwards, instead of the few
+// reversing lanes of a mostly marching wave.  A queue that fills sets
+// qcnt[Q_OVER]; the host then re-runs that chunk of photons in smaller pieces.
 
 __device__ __forceinline__ void adj_overflow(const RenderArgs &A) { atomicMax(A.qcnt + Q_OVER, 1ull); }
 
@@ -375,6 +376,20 @@ __device__ __forceinline__ void copy_records(float *dst, const float *src, int n
     for (int i = 0; i < 4 * n; ++i) d[i] = s[i];
 }
 
+// A main-path slot for the lane's photon (its last vertex with an adjoint starts
+// at none).
+__device__ __forceinline__ void adj_take_slot(Lane &L) {
+    AdjState &a = *L.a;
+    const RenderArgs &A = L.A;
+    const unsigned long long sl = atomicAdd(A.qcnt + Q_SLOTS, 1ull);
+    if (sl >= A.slot_cap) {
+        adj_overflow(A);
+        return;
+    }
+    a.slot = a.jslot = (int)sl;
+    atomicExch(reinterpret_cast<int *>(A.slots + (size_t)sl * 16 + 6), -1);
+}
+
 // Queue the current sub-path's backward run (the state sub_rev_start takes).
 __device__ __forceinline__ void adj_defer_sub(Lane &L, f3 lp, f3 lv, float mu, float ln, int phase) {
     AdjState &a = *L.a;
@@ -382,8 +397,9 @@ __device__ __forceinline__ void adj_defer_sub(Lane &L, f3 lp, f3 lv, float mu, f
     const Hot &h = L.h;
     int slot = -1;
     if (phase == RP_NEE) {
+        if (a.jslot < 0 && L.c.phase == PH_NEE) adj_take_slot(L);  // the lane's own photon
         slot = a.jslot;
-        if (slot < 0) return;  // no slot left: adj_vertex_slot flagged it
+        if (slot < 0) return;  // no slot left: adj_take_slot flagged it
         atomicMax(reinterpret_cast<int *>(A.slots + (size_t)slot * 16 + 6), a.jvert);
     }
     const unsigned long long j = atomicAdd(A.qcnt + Q_JOBS, 1ull);
@@ -412,22 +428,14 @@ __device__ __forceinline__ void adj_defer_sub(Lane &L, f3 lp, f3 lv, float mu, f
                        0.f);
 }
 
-// A vertex of the deferred re-trace with a next-event sub-path to trace: the
-// photon's main-path slot (taken at its first such vertex; its last vertex
-// with an adjoint starts at none) and what the sub-path's job needs to know
-// of it.
-__device__ __forceinline__ void adj_vertex_slot(Lane &L) {
+// A vertex of the deferred re-trace with a next-event sub-path to trace: what
+// the sub-path's job needs to know of its main path.  The sub-paths of a photon
+// that may use the wave's stack (a.push) need its slot at once, since the photon
+// may have ended when they do; any other photon's take it when one touches the
+// objective.
+__device__ __forceinline__ void adj_vertex(Lane &L) {
     AdjState &a = *L.a;
-    const RenderArgs &A = L.A;
-    if (a.slot < 0 && !a.trunc_main) {
-        const unsigned long long sl = atomicAdd(A.qcnt + Q_SLOTS, 1ull);
-        if (sl >= A.slot_cap) {
-            adj_overflow(A);
-        } else {
-            a.slot = (int)sl;
-            atomicExch(reinterpret_cast<int *>(A.slots + (size_t)sl * 16 + 6), -1);
-        }
-    }
+    if (a.push && a.slot < 0 && !a.trunc_main) adj_take_slot(L);
     a.jslot = a.slot;
     a.jvert = a.nmain - 1;
     a.jtrunc = a.trunc_main;
@@ -449,7 +457,7 @@ __device__ __forceinline__ void adj_job_load(Lane &L, float4 r) {
 }
 
 // Photon end of the deferred re-trace: store the main-path log of a photon
-// with traced next-event sub-paths, which may still be on the wave's stack
+// with a slot, whose next-event sub-paths may still be on the wave's stack
 // (slot layout: source, scaling; tau, record count, last vertex with an
 // adjoint -- kept by the sub-paths' jobs -- valid; record base,
 // configuration).

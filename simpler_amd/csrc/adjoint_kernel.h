@@ -270,10 +270,10 @@ __global__ void __launch_bounds__(kBlock) k_adjoint(DevScene S, RenderArgs A) {
 
 // The deferred image adjoint's re-trace: forward runs and logs only, backward
 // runs queued for k_adj_rev (no parameter derivatives here).  The render
-// kernel's loop: next-event sub-paths on the wave's stack, march_chunk, the
-// event code's arguments re-read on every turn.  BATCH: photons of many
-// point-source patterns; a lane's objective sum goes to its pattern's when
-// the lane moves to another one.
+// kernel's loop: the chunk's last photons leave their next-event sub-paths on the
+// wave's stack, march_chunk, the event code's arguments re-read on every turn.
+// BATCH: photons of many point-source patterns; a lane's objective sum goes to
+// its pattern's when the lane moves to another one.
 // A small launch is bound by the chain of its longest photon; before, that was
 // the main path and all its sub-paths, one lane per photon.  Whole adjoint,
 // before -> with this and the spread backward kernels: 2^17 photons of the
@@ -284,6 +284,7 @@ k_retrace(DevScene S0, RenderArgs A0) {
     constexpr int MODE = M_ADJDEF;
     __shared__ Cold cold[kBlock];
     __shared__ uint32_t cnt[C_N];
+    __shared__ float4 mcache[kBlock];
     __shared__ uint32_t nheld[kBlock / 64];  // entries of each wave's next-event stack
     if (threadIdx.x < C_N) cnt[threadIdx.x] = 0u;
     if ((threadIdx.x & 63) == 0) nheld[threadIdx.x >> 6] = 0u;
@@ -297,7 +298,7 @@ k_retrace(DevScene S0, RenderArgs A0) {
     scell.key = -1;
     a.F = 0.0;
     a.rsteps = a.nsubrev = a.nmainrev = a.dropped = 0;
-    a.pending = a.trunc_main = a.trunc_sub = a.jtrunc = false;
+    a.pending = a.trunc_main = a.trunc_sub = a.jtrunc = a.push = false;
     a.slot = a.jslot = -1;
     a.cfg = 0;
     a.gL = 0.f;
@@ -309,7 +310,7 @@ k_retrace(DevScene S0, RenderArgs A0) {
         int tid = (int)threadIdx.x;
         asm volatile("" : "+v"(tid));
         Var vsingle = var_from(S, A);
-        Lane L{h, cold[tid], BATCH ? const_cast<Var *>(A.cfgs) + a.cfg : &vsingle, S, A, cnt, &a, nullptr, nullptr,
+        Lane L{h, cold[tid], BATCH ? const_cast<Var *>(A.cfgs) + a.cfg : &vsingle, S, A, cnt, &a, &mcache[tid], nullptr,
                nullptr, true};
         const size_t gid = (size_t)blockIdx.x * kBlock + tid;
         a.log_main = A.log + gid * (size_t)(A.main_cap + A.sub_cap) * kRecFloats;
@@ -330,6 +331,7 @@ k_retrace(DevScene S0, RenderArgs A0) {
                 L.v = const_cast<Var *>(A.cfgs) + c;
             }
         };
+        a.push |= !left && A.push_from < A.n;  // lanes of the wave are without photons from now on
         unsigned long long need = __ballot(h.state == ST_NEED);
         if (need) {
             const uint32_t held = __builtin_amdgcn_readfirstlane(wave_get(L.qn));
@@ -357,6 +359,7 @@ k_retrace(DevScene S0, RenderArgs A0) {
             if ((need >> lane) & 1ull) {
                 const unsigned long long idx = base + __popcll(need & ((1ull << lane) - 1ull));
                 if (idx < A.n) {
+                    a.push = idx >= A.push_from;
                     uint64_t pid = A.offset + idx;
                     if (BATCH) {  // A.offset + idx: the photon's index over all configurations
                         int c;
@@ -371,7 +374,7 @@ k_retrace(DevScene S0, RenderArgs A0) {
         }
         if (h.state == ST_INIT) photon_init<FIELD, MODE>(L);
         if (h.state == ST_SEG_END) seg_end<FIELD, MODE>(L);
-        if (h.state == ST_NEED && a.slot >= 0) {  // a photon with traced next-event sub-paths ended
+        if (h.state == ST_NEED && a.slot >= 0) {  // a photon with a main-path slot ended
             adj_store_slot(L);
             a.slot = -1;
         }

@@ -102,6 +102,7 @@ struct RenderArgs {
     float *jobs, *jobrec, *slots, *slotrec;
     unsigned long long *qcnt;
     unsigned long long job_cap, jobrec_cap, slot_cap, slotrec_cap;
+    unsigned long long push_from;  // photons of the chunk from this index on may use the re-trace's stacks
     // spline adjoint: one gradient copy per XCD (kXcds copies, gx_stride
     // floats apart), summed into grad by k_gx_reduce
     float *gx;
@@ -1193,9 +1194,14 @@ __device__ __forceinline__ void vertex(Lane &L) {
                 c.stream = 0;
                 c.draw = c.main_draw;
             }
-            if constexpr (MODE == M_ADJDEF)
-                if (!walk_on) adj_vertex_slot(L);
-            walk_on = walk_on || nee_push<FIELD, MODE>(L);
+            if constexpr (MODE == M_ADJDEF) {
+                if (!walk_on) {
+                    adj_vertex(L);
+                    walk_on = L.a->push && nee_push<FIELD, MODE>(L);
+                }
+            } else {
+                walk_on = walk_on || nee_push<FIELD, MODE>(L);
+            }
         }
         if (!walk_on) {
             c.mp = h.p;
@@ -3347,10 +3353,11 @@ static int adjoint_buffers(simpler_ctx *ctx) {
 // sub-paths (128 B each) with c sub-path records, c main paths (64 B) with
 // 8 c main-path records (64 B each): 6 GiB at the default c = 2^23,
 // allocated on first use.  The 64^3 spline scene with scattering queues about
-// 0.6 sub-paths and 0.2 main paths per photon, with a few tens of records
-// each.  The chunk starts at 2^22 photons (a chunk drains like a launch of
-// its own, so larger is faster), halves when a chunk overflows and doubles
-// after a chunk that filled no queue past 40 %; it is kept by the context.
+// 0.6 sub-paths and 0.2 main paths per photon (all of them for the last photons
+// of a chunk, see adjoint_deferred), with a few tens of records each.  The chunk
+// starts at 2^22 photons (a chunk drains like a launch of its own, so larger is
+// faster), halves when a chunk overflows and doubles after a chunk that leaves
+// room for twice its photons; it is kept by the context.
 constexpr int64_t kAdjChunkMin = 1 << 14, kAdjChunkMax = 1 << 24;
 constexpr int kQWords = 32;  // Q_N counters; objective / adjoint counters and event counters backed up at 16, 24
 
@@ -3403,10 +3410,12 @@ static void launch_adj_inline(simpler_ctx *ctx, dim3 grid, const DevScene &S, co
 // The image adjoint in chunks of photons: re-trace (queueing the backward
 // runs), then the queued sub-paths, then the stored main paths.  A chunk whose
 // queues overflow has its objective and counters restored and is re-traced
-// as a chunk half its size; at the smallest chunk it runs with the backward
-// runs inline.  BATCH: photons of a pattern batch, indexed over all its
-// configurations; their objectives (n_obj doubles at A.obj) are backed up
-// in obj_backup for each chunk.
+// as a chunk half its size; from the smallest such chunk on the photons run with
+// the backward runs inline, in one launch (2^17 photons of the 64^3 spline scene
+// with queues of 2^12: chunk by chunk 2.52 s, in one launch 0.51).  BATCH:
+// photons of a pattern batch, indexed over all its configurations; their
+// objectives (n_obj doubles at A.obj) are backed up in obj_backup for each
+// chunk.
 template <int F, bool BATCH = false>
 static int adjoint_deferred(simpler_ctx *ctx, dim3 grid, const DevScene &S, RenderArgs A, int64_t n,
                             size_t n_obj = 0, double *obj_backup = nullptr) {
@@ -3426,17 +3435,24 @@ static int adjoint_deferred(simpler_ctx *ctx, dim3 grid, const DevScene &S, Rend
     A.nq_waves = (int)tgrid.x * (kBlock / 64);
     A.nq_cap = (int)std::min<size_t>(kStackEntries, (size_t)ctx->nq_waves * kStackEntries * job_vec(M_RENDER) /
                                                         ((size_t)A.nq_waves * job_vec(M_ADJDEF)));
-    // every photon with a next-event sub-path to trace stores its main path:
-    // a vertex per mean free path of the block and a few faces (more photons
-    // per chunk than their records fit would only be traced twice)
+    // A photon with a sub-path on a stack stores its main path, whether its
+    // sub-paths touch the objective or not (adj_vertex).  The stacks serve lanes
+    // without photons, so only a chunk's last photons use them, and those still
+    // marching when the last is taken: so many that their records (a vertex per
+    // mean free path of the block and a few faces) take half the queues, and
+    // none where these hold fewer than a launch's lanes.  When all photons used
+    // them, nearly all main paths were stored instead of one in five, and 2^22
+    // photons of the 64^3 spline scene took three chunks: 2.49 s -> 2.18.
     const double rec = 6.0 + 1.5 * (double)S.sigma_t * (double)(S.blockR.x - S.blockL.x);
-    const int64_t fit = std::max<int64_t>(kAdjChunkMin, (int64_t)(0.9 * (double)A.slotrec_cap / rec));
+    const int64_t lanes = (int64_t)tgrid.x * kBlock;
+    const int64_t push_last = (int64_t)(0.5 * std::min((double)A.slot_cap, (double)A.slotrec_cap / rec));
     const double caps[4] = {(double)A.job_cap, (double)A.jobrec_cap, (double)A.slot_cap, (double)A.slotrec_cap};
     int64_t start = 0;
     while (start < n) {
-        const int64_t m = std::min<int64_t>(std::min<int64_t>(ctx->adj_chunk, fit), n - start);
+        int64_t m = std::min<int64_t>(ctx->adj_chunk, n - start);
         A.offset = off0 + (uint64_t)start;
         A.n = (uint64_t)m;
+        A.push_from = (uint64_t)(push_last < std::min(m, lanes) ? m : std::max<int64_t>(0, m - push_last));
         A.wave_photons = wave_share(A.n, (uint64_t)tgrid.x * (kBlock / 64));
         HIP_TRY(ctx, hipMemcpyAsync(ctx->d_q + 16, ctx->d_adj, 8 * sizeof(unsigned long long),
                                     hipMemcpyDeviceToDevice, ctx->cur));
@@ -3463,14 +3479,22 @@ static int adjoint_deferred(simpler_ctx *ctx, dim3 grid, const DevScene &S, Rend
                 ctx->adj_chunk = std::max<int64_t>(kAdjChunkMin, m / 2);
                 continue;
             }
+            // queues too small for any chunk: the rest of the photons inline
+            m = n - start;
+            A.n = (uint64_t)m;
             hipLaunchKernelGGL(k_fill_u64, dim3(1), dim3(64), 0, ctx->cur, ctx->d_scratch, 1);
             launch_adj_inline<F, BATCH>(ctx, grid, S, A);
         } else {
             hipLaunchKernelGGL((k_adj_rev<F, M_ADJSUB, BATCH>), rgrid, dim3(kBlock), 0, ctx->cur, S, A);
             hipLaunchKernelGGL((k_adj_rev<F, M_ADJMAIN, BATCH>), rgrid, dim3(kBlock), 0, ctx->cur, S, A);
-            double fill = 0.0;
-            for (int k = 0; k < 4; ++k) fill = std::max(fill, (double)q[k] / caps[k]);
-            if (m == ctx->adj_chunk && fill < 0.4 && ctx->adj_chunk < kAdjChunkMax) ctx->adj_chunk *= 2;
+            // a chunk of 2 m fills the queues twice as far, but for the main
+            // paths of the photons that use the stacks
+            const double pushed = (double)(A.n - A.push_from);
+            double fill = std::max((double)q[Q_JOBS] / caps[0], (double)q[Q_JOBREC] / caps[1]) * 2.0;
+            fill = std::max(fill, (2.0 * (double)q[Q_SLOTS] - pushed) / caps[2]);
+            if (q[Q_SLOTS])
+                fill = std::max(fill, (2.0 - pushed / (double)q[Q_SLOTS]) * (double)q[Q_SLOTREC] / caps[3]);
+            if (m == ctx->adj_chunk && fill < 0.8 && ctx->adj_chunk < kAdjChunkMax) ctx->adj_chunk *= 2;
         }
         HIP_TRY(ctx, hipGetLastError());
         start += m;
