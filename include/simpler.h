@@ -456,10 +456,9 @@ int simpler_adjoint_rays(simpler_scene *scene, int64_t n_rays, uint64_t seed,
  * block_size in {64,128,256} (the kernels are compiled for at most 256
  * lanes per workgroup), steps_per_chunk in [1,4096] (march steps between
  * event phases), blocks_per_cu in [1,64].  0 keeps the current value; other
- * values fail with SIMPLER_ERR_INVALID.  Renders of a context on which neither
- * this call (with a non-zero value) nor the autotuner has chosen a shape pick
- * their grid and steps per event phase by their photon count and field;
- * get_tuning then reports the defaults. */
+ * values fail with SIMPLER_ERR_INVALID.  At the defaults (256, 32, 4) renders
+ * pick their grid and steps per event phase by their photon count and field;
+ * setting them again restores that.  Other values are taken as they are. */
 int simpler_ctx_set_tuning(simpler_ctx *ctx, int block_size,
                            int steps_per_chunk, int blocks_per_cu);
 int simpler_ctx_get_tuning(simpler_ctx *ctx, int *block_size,

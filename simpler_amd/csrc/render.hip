@@ -58,6 +58,7 @@ enum { Q_JOBS = 0, Q_JOBREC, Q_SLOTS, Q_SLOTREC, Q_OVER, Q_WSUB, Q_WMAIN, Q_N };
 enum { C_PHOT = 0, C_STEPS, C_SCAT, C_NEE, C_DIRECT, C_FACE, C_SEG, C_ABORT, C_N };
 constexpr uint32_t kMaxFaceEvents = 1u << 20;  // per march; see the abort counter
 constexpr int kBlock = 256;
+constexpr int kSpc = 32, kBpc = 4;  // default march steps per event phase, workgroups per CU
 constexpr int kJtabLds = 128;  // Bessel table intervals staged in LDS (8 KiB)
 constexpr int kJtabLdsBatch = 1024;  // float4 (16 KiB): a batch's per-order tables in LDS
 constexpr int kMaxMode = 7;          // highest Bessel order (check_desc)
@@ -1919,8 +1920,7 @@ struct simpler_ctx {
     float4 *d_nq = nullptr;  // next-event stacks of the first nq_waves waves of a render grid
     int nq_waves = 0;
     int num_cu = 256;
-    int block = 256, spc = 32, bpc = 4;
-    bool shape_set = false;  // chosen by the caller or the autotuner: renders take it as it is
+    int block = kBlock, spc = kSpc, bpc = kBpc;  // at these values renders choose their shape (auto_shape)
     int splat = 0;  // splat strategy: 0 per-lane atomics, 1 wave-aggregated
     int live = 0;  // scenes and batches not yet destroyed
     float *d_log = nullptr;  // adjoint segment logs (grown on demand)
@@ -2245,6 +2245,13 @@ static int wave_share(uint64_t n, uint64_t waves) {
     return (int)std::max<uint64_t>(1, std::min<uint64_t>(64, (n + waves - 1) / waves));
 }
 
+// The default tuning stands for the shape that render_shape chooses, also in
+// the autotuner's candidates: whoever sets a tuning that get_tuning returned has
+// the launches that it had.
+static bool auto_shape(const simpler_ctx *ctx) {
+    return ctx->block == kBlock && ctx->spc == kSpc && ctx->bpc == kBpc;
+}
+
 // A render's grid, march steps per event phase and wave_share.  Where the
 // caller (or the autotuner) has chosen a launch shape it is taken as it is.
 // Otherwise a launch takes as many workgroups of 256 as give each wave eight
@@ -2259,7 +2266,7 @@ static int wave_share(uint64_t n, uint64_t waves) {
 // photons 414 -> 364 ms, 4,096 spline photons 40.8 -> 31.4 ms, 2^17 142 -> 136 ms,
 // 4,096 photons of 16 sources 111 -> 55 ms, 2^15 135 -> 119 ms, 2^17 242 -> 216 ms.
 static void render_shape(const simpler_ctx *ctx, RenderArgs &A, int &blocks, int field, bool batch) {
-    if (ctx->shape_set) {
+    if (!auto_shape(ctx)) {
         blocks = std::max(1, ctx->num_cu * ctx->bpc);
     } else {
         const bool bessel = field == SIMPLER_FIELD_BESSEL;
@@ -2505,7 +2512,6 @@ int simpler_ctx_set_tuning(simpler_ctx *ctx, int block_size, int steps_per_chunk
         if (blocks_per_cu < 1 || blocks_per_cu > 64) return fail(ctx, SIMPLER_ERR_INVALID, "blocks_per_cu out of range [1,64]");
         ctx->bpc = blocks_per_cu;
     }
-    ctx->shape_set |= block_size || steps_per_chunk || blocks_per_cu;
     return SIMPLER_OK;
 }
 
@@ -2540,8 +2546,6 @@ int simpler_autotune(simpler_scene *sc, int64_t n_photons, int X, int Y, int Z, 
     float best_ms = INFINITY;
     rc = SIMPLER_OK;
     bool warm = false;
-    const bool was_set = ctx->shape_set;
-    ctx->shape_set = true;
     // launch shapes with per-lane splats, then the aggregated splat at the
     // best shape (the strategy changes the event phase, not the march)
     for (int stage = 0; stage < (has_agg ? 2 : 1); ++stage)
@@ -2580,7 +2584,6 @@ int simpler_autotune(simpler_scene *sc, int64_t n_photons, int X, int Y, int Z, 
     ctx->spc = best[1];
     ctx->bpc = best[2];
     ctx->splat = best[3];
-    ctx->shape_set = was_set || best_ms < INFINITY;
     (void)hipEventDestroy(e0);
     (void)hipEventDestroy(e1);
     (void)hipFree(img);
