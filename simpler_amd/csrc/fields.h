@@ -114,6 +114,34 @@ template <int FIELD>
 __device__ __forceinline__ void field_eval(const DevScene &S, const FieldP &F, f3 p, float scaling, float tau,
                                            float &n, f3 &g);
 
+// One turn of the angle-addition recurrence, (cm, sm) rotated by (c1, s1), and
+// the gradient cr rho + ctan (uz x rho, or the component form's), used by every
+// Bessel evaluation with its additions fused by hand, in the order that the
+// compiler had chosen: which evaluation a step runs follows from the other lanes
+// of its wave, so they must not differ in a bit.
+__device__ __forceinline__ void angle_add(float &cm, float &sm, float c1, float s1) {
+    const float cn = __builtin_fmaf(cm, c1, -(sm * s1));
+    sm = __builtin_fmaf(cm, s1, sm * c1);
+    cm = cn;
+}
+template <int MM, int GA>
+__device__ __forceinline__ f3 bessel_grad(const DevScene &S, bool general, f3 rho, float cr, float ctan) {
+    if (MM == 0) {
+        if (GA == 2) return mk3(cr * rho.x, cr * rho.y, 0.f);
+        return general ? cr * rho : mk3(0.f, cr * rho.y, cr * rho.z);
+    }
+    if (GA == 2)
+        return mk3(__builtin_fmaf(ctan, rho.y, cr * rho.x), __builtin_fmaf(cr, rho.y, -(ctan * rho.x)), 0.f);
+    if (general) {
+        const f3 u = S.uz;
+        const f3 tp = f3{__builtin_fmaf(u.y, rho.z, -(u.z * rho.y)), __builtin_fmaf(u.z, rho.x, -(u.x * rho.z)),
+                         __builtin_fmaf(u.x, rho.y, -(u.y * rho.x))};
+        return f3{__builtin_fmaf(cr, rho.x, -(ctan * tp.x)), __builtin_fmaf(cr, rho.y, -(ctan * tp.y)),
+                  __builtin_fmaf(cr, rho.z, -(ctan * tp.z))};
+    }
+    return mk3(0.f, __builtin_fmaf(cr, rho.y, -(ctan * rho.z)), __builtin_fmaf(ctan, rho.y, cr * rho.z));
+}
+
 // reference scene.cpp:205-257 (axis = +-x component form) or the same
 // gradient for a general axis: grad n = A s [J'(kr) k cos(m phi) rho/r
 //                                           - J m sin(m phi) (uz x rho)/r^2]
@@ -159,11 +187,7 @@ __device__ __forceinline__ void bessel_eval(const DevScene &S, const FieldP &F, 
             sm = s1;
         }
 #pragma unroll
-        for (int k = MM > 0 ? 1 : 0; k < (MM >= 0 ? MM : mode); ++k) {
-            const float cn = cm * c1 - sm * s1;
-            sm = sm * c1 + cm * s1;
-            cm = cn;
-        }
+        for (int k = MM > 0 ? 1 : 0; k < (MM >= 0 ? MM : mode); ++k) angle_add(cm, sm, c1, s1);
     }
     float J, dJ;
     const bool clamp = r < kEps;
@@ -186,22 +210,7 @@ __device__ __forceinline__ void bessel_eval(const DevScene &S, const FieldP &F, 
     bessel_tab(F, F.k_r * r, J, dJ);
     if (!clamp) n = S.n_o + A * J * cm;
     const float cr = (A * F.k_r) * dJ * ir * cm;
-    if (MM == 0) {
-        if (GA == 2)
-            g = mk3(cr * rho.x, cr * rho.y, 0.f);
-        else
-            g = general ? cr * rho : mk3(0.f, cr * rho.y, cr * rho.z);
-        return;
-    }
-    const float ctan = A * J * (float)mode * sm * ir * ir;
-    if (GA == 2) {
-        g = mk3(cr * rho.x + ctan * rho.y, cr * rho.y - ctan * rho.x, 0.f);
-    } else if (general) {
-        const f3 tp = cross(S.uz, rho);
-        g = mk3(cr * rho.x - ctan * tp.x, cr * rho.y - ctan * tp.y, cr * rho.z - ctan * tp.z);
-    } else {
-        g = mk3(0.f, cr * rho.y - ctan * rho.z, cr * rho.z + ctan * rho.y);
-    }
+    g = bessel_grad<MM, GA>(S, general, rho, cr, A * J * (float)mode * sm * ir * ir);
 }
 
 // bessel_eval at a point away from the axis (r2, the square of the distance
@@ -238,32 +247,13 @@ __device__ __forceinline__ void bessel_eval_far(const DevScene &S, const FieldP 
             sm = s1;
         }
 #pragma unroll
-        for (int k = MM > 0 ? 1 : 0; k < (MM >= 0 ? MM : mode); ++k) {
-            const float cn = cm * c1 - sm * s1;
-            sm = sm * c1 + cm * s1;
-            cm = cn;
-        }
+        for (int k = MM > 0 ? 1 : 0; k < (MM >= 0 ? MM : mode); ++k) angle_add(cm, sm, c1, s1);
     }
     float J, dJ;
     bessel_tab(F, F.k_r * r, J, dJ);
     n = S.n_o + A * J * cm;
     const float cr = (A * F.k_r) * dJ * ir * cm;
-    if (MM == 0) {
-        if (GA == 2)
-            g = mk3(cr * rho.x, cr * rho.y, 0.f);
-        else
-            g = general ? cr * rho : mk3(0.f, cr * rho.y, cr * rho.z);
-        return;
-    }
-    const float ctan = A * J * (float)mode * sm * ir * ir;
-    if (GA == 2) {
-        g = mk3(cr * rho.x + ctan * rho.y, cr * rho.y - ctan * rho.x, 0.f);
-    } else if (general) {
-        const f3 tp = cross(S.uz, rho);
-        g = mk3(cr * rho.x - ctan * tp.x, cr * rho.y - ctan * tp.y, cr * rho.z - ctan * tp.z);
-    } else {
-        g = mk3(0.f, cr * rho.y - ctan * rho.z, cr * rho.z + ctan * rho.y);
-    }
+    g = bessel_grad<MM, GA>(S, general, rho, cr, A * J * (float)mode * sm * ir * ir);
 }
 
 template <>

@@ -1,0 +1,62 @@
+"""A march step with a rare case anywhere in its wave evaluates the Bessel field
+by another function than one without, so a path must not depend on which:
+recorded rays have the same bits in shards of a call and under launch shapes
+that put other rays into their waves, and a batch takes the steps of its
+configurations rendered alone where both evaluate the same form of the field
+(along z a single scene has kernels of the axis frame for orders 0 and 2 only).
+"""
+import pytest
+import torch
+
+from simpler_amd import engine, scenes
+
+pytestmark = pytest.mark.gpu
+
+AXES = {
+    "z": dict(),
+    "x": dict(axis_uz=(-1.0, 0.0, 0.0), axis_ux=(0.0, 0.0, 1.0)),
+    "oblique": dict(axis_uz=(0.48, 0.6, 0.64), axis_ux=(0.8, 0.0, -0.6)),
+    "component": dict(axis_uz=(-1.0, 0.0, 0.0), axis_ux=(0.0, 0.0, 1.0),
+                      flags=scenes.FLAGS_DEFAULT & ~scenes.FLAG_GENERAL_AXIS),
+}
+
+
+@pytest.mark.parametrize("axis", list(AXES))
+@pytest.mark.parametrize("mode", [0, 1, 2, 3, 7])
+def test_rays_do_not_depend_on_their_wave(axis, mode):
+    ctx = engine.Context(0)
+    d, tex, _ = scenes.transparent_cube(mode=mode, step=5e-5)
+    d.set(n_max=2e-3, n_clip=2e-3, **AXES[axis])
+    sc = engine.Scene(ctx, d, tex)
+    n = 20000
+    ref = sc.trace_rays(n, seed=5)
+    for off in (1, 17, 1000):
+        for a, b in zip(ref, sc.trace_rays(n - off, seed=5, offset=off)):
+            assert torch.equal(a[off:], b), off
+    for shape in ((64, 16, 1), (128, 7, 3)):
+        ctx.set_tuning(*shape)
+        for a, b in zip(ref, sc.trace_rays(n, seed=5)):
+            assert torch.equal(a, b), shape
+    sc.close()
+    ctx.close()
+
+
+@pytest.mark.parametrize("axis,modes", [("z", [0, 2, 2]), ("x", [0, 1, 2, 3, 5]), ("oblique", [0, 1, 2, 3, 5])])
+def test_batch_takes_the_steps_of_its_configurations(gpu_ctx, axis, modes):
+    d, tex, cfgs, _ = scenes.batched_configs(n_cfg=len(modes), seed=4)
+    d.set(er_stepsize=2e-5, **AXES[axis])
+    for c, m in zip(cfgs, modes):
+        c["mode"], c["n_photons"] = m, 10000
+    base = engine.Scene(gpu_ctx, d, tex)
+    b = engine.Batch(base, cfgs, (16, 16, 8))
+    _, st = b.render()
+    b.close()
+    total = dict.fromkeys(st, 0)
+    for c in cfgs:
+        sc = engine.Scene(gpu_ctx, scenes.desc_for_config(d, c), tex)
+        _, s1 = sc.render(c["n_photons"], (16, 16, 8), seed=c["seed"])
+        sc.close()
+        for k in total:
+            total[k] += s1[k]
+    base.close()
+    assert st == total
