@@ -5,9 +5,11 @@ that put other rays into their waves, and a batch takes the steps of its
 configurations rendered alone where both evaluate the same form of the field
 (along z a single scene has kernels of the axis frame for orders 0 and 2 only).
 """
+import numpy as np
 import pytest
 import torch
 
+from oracle import oracle as O
 from simpler_amd import engine, scenes
 
 pytestmark = pytest.mark.gpu
@@ -60,3 +62,21 @@ def test_batch_takes_the_steps_of_its_configurations(gpu_ctx, axis, modes):
             total[k] += s1[k]
     base.close()
     assert st == total
+
+
+@pytest.mark.parametrize("axis", list(AXES))
+@pytest.mark.parametrize("mode", [0, 1, 4])
+def test_few_rays_match_the_oracle(gpu_ctx, axis, mode):
+    """13 rays: the loop of waves with few marching lanes, against FP64."""
+    d, tex, _ = scenes.transparent_cube(mode=mode, step=2e-5)
+    d.set(**AXES[axis])
+    sc = engine.Scene(gpu_ctx, d, tex)
+    p, dr, L, s = (t.double().cpu().numpy() for t in sc.trace_rays(13, seed=6))
+    sc.close()
+    po, do, Lo, so = O.OracleScene(d, tex).trace_rays(13, seed=6, precision=64)[:4]
+    assert np.array_equal(s, so) and (s == 1).sum() > 0
+    k = s == 1
+    # 1e-5 relative: of the half width (5 mm), of 1, of L
+    assert np.abs(p[k] - po[k]).max() < 5e-8
+    assert np.abs(dr[k] - do[k]).max() < 1e-5
+    assert (np.abs(L[k] - Lo[k]) / Lo[k]).max() < 1e-5
