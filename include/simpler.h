@@ -153,7 +153,9 @@ void simpler_scene_desc_default(simpler_scene_desc *desc);
 
 /* ---- context: one device + one HIP stream; calls on one ctx are not
  *      thread-safe, separate ctx objects are independent.  Replaces the
- *      process-global __constant__ state of cuda_renderer.cu:28-48. ------ */
+ *      process-global __constant__ state of cuda_renderer.cu:28-48.  A
+ *      context holds the next-event stacks of its launches from its
+ *      creation, 80 KiB of device memory per CU (20 MiB on 256 CUs). ------ */
 int simpler_ctx_create(int device, simpler_ctx **out);
 /* Fails with SIMPLER_ERR_STATE while scenes or batches of the context are
  * alive (destroy them first); scene_destroy likewise fails while batches

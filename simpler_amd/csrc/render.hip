@@ -400,7 +400,10 @@ __device__ __forceinline__ unsigned long long not_ordinary(const DevScene &S, f3
            __builtin_amdgcn_ballot_w64(!(p.z > S.inL.z)) | __builtin_amdgcn_ballot_w64(!(p.z < S.inR.z));
 }
 
-constexpr int kFewLanes = 20;  // marching lanes of a wave up to which ordinary steps get a loop of their own
+// Marching lanes of a wave up to which ordinary steps get a loop of their own.
+// With 0 / 8 / 20 / 32 / 64: 64 photons 4.0 / 3.6 / 3.5 / 3.5 / 3.4 ms, 5,000
+// photons 7.5 / 6.3 / 5.9 / 5.9 / 5.9, 2^22 photons 371 / 366 / 364 / 364 / 408.
+constexpr int kFewLanes = 20;
 
 // One ordinary march step (see march_chunk) of the lanes of a wave: false, and
 // nothing changed, when some lane's step is not certain to be one.
@@ -1173,9 +1176,8 @@ __device__ __forceinline__ void nee_pop(Lane &L, uint32_t i) {
 }
 
 // photon.cpp:111-116 loop head + scene.cpp:866-893 (NEE start).  Forward
-// renders take nee_skip in the spline kernels only: inlined into the Bessel
-// kernel's event code it slows that kernel's march loop by a fifth per step,
-// more than the 11 % of its steps it removes.
+// renders take nee_skip in the spline kernels only.  (In the Bessel kernels it
+// would remove 10.8 % of the steps: 2^22 photons 364 -> 344 ms.)
 template <int FIELD, int MODE>
 __device__ __forceinline__ void vertex(Lane &L) {
     const DevScene &S = L.S;
@@ -1531,9 +1533,10 @@ __device__ __forceinline__ uint64_t batch_photon(const RenderArgs &A, unsigned l
 // that the compiler takes for new at each call, so that what is read through
 // it is loaded where it is used and not kept in registers.  Read as plain
 // arguments, 150 scalars were spilled to vector registers and 45 vectors to
-// scratch in the m = 0 kernel (0 and 2 now), and the batched kernels fit three
-// waves per SIMD instead of four: 2^22 photons 447 -> 413 ms, the
-// 256-configuration sweep 391 -> 362 ms, 2^17 spline photons 172 -> 141 ms.
+// scratch in the m = 0 kernel (now 6 and 2; m = 2: 6 and 22, in the event code),
+// and the batched kernels fit three waves per SIMD instead of four: 2^22 photons
+// 447 -> 413 ms, the 256-configuration sweep 391 -> 362 ms, 2^17 spline photons
+// 172 -> 141 ms.
 template <class T>
 __device__ __forceinline__ const T &kernel_arg(size_t offset) {
     using Segment = const __attribute__((address_space(4))) char *;
@@ -1622,7 +1625,7 @@ __device__ __forceinline__ void render_order(const DevScene &S0, const RenderArg
 // on its order where one exists (m <= 2).  A wave goes on to the next group as
 // soon as it finds no more work in its own; as one launch per order, each
 // waited for the longest photons of the one before: 256 configurations of
-// three orders, 7.1e10 steps 354 -> 257 ms.
+// three orders, 7.1e10 steps 354 -> 257 ms (other seeds' budgets: 257 to 290).
 __global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4)))
 k_render_orders(DevScene S0, RenderArgs A0) {
     __shared__ Cold cold[kBlock];
