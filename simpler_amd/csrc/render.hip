@@ -2263,18 +2263,25 @@ static bool auto_shape(const simpler_ctx *ctx) {
 // the longest photon's down, and fewer leave SIMDs idle.  hi is what the kernel
 // keeps resident (five for single Bessel scenes, four for their batches, two
 // for the spline's 256 registers), and two for point sources, whose long step
-// two waves per SIMD fill.  A Bessel launch with many photons for every lane
-// also takes 128 steps per event phase.  Measured, the fixed four workgroups
-// per CU and 32 steps -> this rule: 16,384 Bessel photons 13.4 -> 11.0 ms, 2^22
-// photons 414 -> 364 ms, 4,096 spline photons 40.8 -> 31.4 ms, 2^17 142 -> 136 ms,
-// 4,096 photons of 16 sources 111 -> 55 ms, 2^15 135 -> 119 ms, 2^17 242 -> 216 ms.
-static void render_shape(const simpler_ctx *ctx, RenderArgs &A, int &blocks, int field, bool batch) {
+// two waves per SIMD fill, or the resident four where so many photons share a
+// lane (the more, the longer the step) that the launch does not last as long as
+// one chain.  A Bessel launch with many photons for every lane also takes 128
+// steps per event phase.  Measured, the fixed four workgroups per CU and 32 steps
+// -> this rule: 16,384 Bessel photons 13.4 -> 11.0 ms, 2^22 photons 414 -> 364 ms,
+// 4,096 spline photons 40.8 -> 31.4 ms, 2^17 142 -> 136 ms, 4,096 photons of 16
+// sources 111 -> 55 ms, 2^15 135 -> 119 ms, 2^17 242 -> 216 ms.  Two -> four
+// workgroups per CU (10 um step), sigma_s 2/mm: 1 source 2^20 photons 214 -> 139 ms,
+// 16 sources 2^17 117 -> 128, 2^18 193 -> 193, 2^20 606 -> 541; sigma_s 0.1/mm: 4
+// sources 2^18 18 -> 21 ms, 2^20 37 -> 34, 16 sources 2^20 85 -> 94, 2^21 139 -> 141.
+static void render_shape(const simpler_ctx *ctx, RenderArgs &A, int &blocks, int field, int n_src, bool batch) {
     if (!auto_shape(ctx)) {
         blocks = std::max(1, ctx->num_cu * ctx->bpc);
     } else {
         const bool bessel = field == SIMPLER_FIELD_BESSEL;
         const uint64_t cus = (uint64_t)std::max(1, ctx->num_cu);
-        const uint64_t lo = bessel ? 2 : 1, hi = bessel ? (batch ? 4 : 5) : 2;
+        // 2^18 photons on 256 CUs for each source, four at least
+        const bool full = field == SIMPLER_FIELD_SOURCES && A.n >= 4 * kBlock * cus * std::max(4, n_src);
+        const uint64_t lo = bessel ? 2 : 1, hi = bessel ? (batch ? 4 : 5) : (full ? 4 : 2);
         const uint64_t want = (A.n + 31) / 32;  // four waves of eight photons
         blocks = (int)std::min(hi * cus, std::max(lo * cus, want));
         if (bessel && !batch && A.n >= 4 * 256 * hi * cus) A.spc = std::max(A.spc, 128);
@@ -2320,7 +2327,7 @@ static void launch_shared_sources(simpler_ctx *ctx, dim3 grid, dim3 block, DevSc
 template <int MODE>
 static void launch_render(simpler_ctx *ctx, int field, const DevScene &S, RenderArgs A) {
     int blocks = std::max(1, ctx->num_cu * ctx->bpc);
-    if (MODE == M_RENDER) render_shape(ctx, A, blocks, field, false);
+    if (MODE == M_RENDER) render_shape(ctx, A, blocks, field, S.n_src, false);
     const dim3 grid(blocks), block(ctx->block);
     switch (field) {
         case SIMPLER_FIELD_BESSEL:
@@ -3751,7 +3758,7 @@ static int batch_launch(simpler_batch *b, float *images, int accumulate, hipStre
     }
     if (b->total > 0) {
         int blocks = 0;
-        render_shape(ctx, A, blocks, b->field, true);
+        render_shape(ctx, A, blocks, b->field, b->S.n_src, true);
         if (b->field == SIMPLER_FIELD_SOURCES)
             hipLaunchKernelGGL((k_render<kSources, M_RENDER, true>), dim3(blocks), dim3(ctx->block), 0, stream, b->S,
                                A);

@@ -1,5 +1,6 @@
 """Setting a tuning that get_tuning returned leaves a context with the launches
-it had: the automatic shape after another one, and a chosen one.
+it had: the automatic shape after another one, and a chosen one; and the
+automatic shape of point sources on both sides of its photon limits.
 """
 import json
 
@@ -40,5 +41,20 @@ def test_tuning_restored(tmp_path):
     assert _shape(sc, n, path) == auto
     ctx.set_tuning(again["block_size"], again["steps_per_chunk"], again["blocks_per_cu"])
     assert _shape(sc, n, path) == chosen
+    sc.close()
+    ctx.close()
+
+
+# 256 CUs: two workgroups per CU, four from 2^18 photons for each of at least
+# four sources on
+@pytest.mark.parametrize("n_src,n,per_cu", [(1, (1 << 20) - 1, 2), (1, 1 << 20, 4), (5, 1 << 20, 2),
+                                            (5, 5 << 18, 4)])
+def test_many_photons_of_few_sources_fill_the_waves(tmp_path, n_src, n, per_cu):
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    ctx = engine.Context(0)
+    d, tex, _, src = scenes.travelling_wave_cube(n_src=n_src, step=1e-3)
+    sc = engine.Scene(ctx, d, tex, sources=src)
+    groups = _shape(sc, n * cus // 256, tmp_path / "trace.json")[0]
+    assert groups == per_cu * cus
     sc.close()
     ctx.close()
