@@ -1565,7 +1565,9 @@ namespace simpler {
 // the few spills fall in the event code), measured 3-6 % faster than 4 waves;
 // five of its workgroups must also fit the CU's 160 KiB of LDS (checked
 // below: 12 more bytes of cold state per lane once cost it a wave per SIMD
-// and 9 % of the render rate).  The spline kernels run 2 waves per SIMD with
+// and 9 % of the render rate).  The forward-mode kernel at 4 (tangents: at 5 it
+// spills 85 registers in its march loop instead of 37; 100 rays of order 0 0.88
+// -> 0.57 ms, 1e6 rays 4.5 -> 3.1).  The spline kernels run 2 waves per SIMD with
 // the current cell's 64 taps in registers (SplineCell); the point-source
 // kernels keep the registers their evaluation needs.
 // MM: the Bessel order when it is known at launch (single-scene renders of
@@ -1578,7 +1580,7 @@ static_assert(5 * (sizeof(Cold) * kBlock + sizeof(uint32_t) * (C_N + kBlock / 64
               "five single-scene Bessel workgroups must fit one CU's LDS");
 
 template <int FIELD, int MODE, bool BATCH, bool JLDS = false, int MM = -1, int GA = -1, int SPLAT = 0>
-__global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(FIELD == kBessel ? 5 : (FIELD == kSpline ? 2 : (FIELD > kSplitSources ? 4 : 1)))))
+__global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(FIELD == kBessel ? (MODE == M_JVP ? 4 : 5) : (FIELD == kSpline ? 2 : (FIELD > kSplitSources ? 4 : 1)))))
 k_render(DevScene S0, RenderArgs A0) {
     __shared__ Cold cold[kBlock];
     __shared__ uint32_t cnt[C_N];
