@@ -1575,11 +1575,12 @@ namespace simpler {
 // reference's axis = x form).
 // SPLAT: 0 = every lane issues its splat's atomics, 1 = wave-aggregated
 // splats (wave_splat after the event phase); an autotuner candidate.
+// STEPS: march_step's loop instead of march_chunk's (see narrow_gap).
 static_assert(5 * (sizeof(Cold) * kBlock + sizeof(uint32_t) * (C_N + kBlock / 64) + sizeof(float4) * (4 * kJtabLds + kBlock)) <=
                   160 * 1024,
               "five single-scene Bessel workgroups must fit one CU's LDS");
 
-template <int FIELD, int MODE, bool BATCH, bool JLDS = false, int MM = -1, int GA = -1, int SPLAT = 0>
+template <int FIELD, int MODE, bool BATCH, bool JLDS = false, int MM = -1, int GA = -1, int SPLAT = 0, bool STEPS = false>
 __global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(FIELD == kBessel ? (MODE == M_JVP ? 4 : 5) : (FIELD == kSpline ? 2 : (FIELD > kSplitSources ? 4 : 1)))))
 k_render(DevScene S0, RenderArgs A0) {
     __shared__ Cold cold[kBlock];
@@ -1617,7 +1618,7 @@ __device__ __forceinline__ void render_order(const DevScene &S0, const RenderArg
                                              const float4 *jlds, float4 *mcache, uint32_t *nheld, int group,
                                              unsigned long long &wave_steps) {
     constexpr int FIELD = kBessel, MODE = M_RENDER, GA = 2, SPLAT = 0;
-    constexpr bool BATCH = true, JLDS = true, STACK = true, SPLIT = false, GROUPS = true;
+    constexpr bool BATCH = true, JLDS = true, STACK = true, SPLIT = false, GROUPS = true, STEPS = false;
     uint32_t *const uncounted = nullptr;
 #include "render_loop.inl"
 }
@@ -2326,6 +2327,14 @@ static void launch_shared_sources(simpler_ctx *ctx, dim3 grid, dim3 block, DevSc
 #undef SIMPLER_RAYS
 }
 
+// Do the gap planes leave less than 0.4 of the block's width between them?  Past
+// them every step takes the rare branch of march_chunk, and recorded rays that
+// fill the launch's lanes run march_step's loop instead: 1e6 rays, a tenth of the
+// block between the planes, m = 0 / 2 / 5: march_chunk 6.7 / 7.5 / 7.9 ms, march_step
+// 5.8 / 6.7 / 7.5; three tenths 6.3 / 6.8 / 7.5 and 5.8 / 6.6 / 7.5; 65,536 rays,
+// a quarter of the lanes, 1.35 / 1.54 / 1.63 and 1.43 / 1.66 / 1.82.
+static bool narrow_gap(const DevScene &S) { return !(S.ord_hi - S.ord_lo >= 0.4f * (S.inR.x - S.inL.x)); }
+
 template <int MODE>
 static void launch_render(simpler_ctx *ctx, int field, const DevScene &S, RenderArgs A) {
     int blocks = std::max(1, ctx->num_cu * ctx->bpc);
@@ -2352,6 +2361,13 @@ static void launch_render(simpler_ctx *ctx, int field, const DevScene &S, Render
                     SIMPLER_RENDER_BV(2, 2, 1)
 #undef SIMPLER_RENDER_BV
                 }
+            } else if (MODE == M_RECORD && A.n >= (uint64_t)blocks * block.x && narrow_gap(S)) {
+                if (S.jtab_n <= kJtabLds)
+                    hipLaunchKernelGGL((k_render<kBessel, M_RECORD, false, true, -1, -1, 0, true>), grid, block, 0,
+                                       ctx->cur, S, A);
+                else
+                    hipLaunchKernelGGL((k_render<kBessel, M_RECORD, false, false, -1, -1, 0, true>), grid, block, 0,
+                                       ctx->cur, S, A);
             } else if (S.jtab_n <= kJtabLds)
                 hipLaunchKernelGGL((k_render<kBessel, MODE, false, true>), grid, block, 0, ctx->cur, S, A);
             else

@@ -1,7 +1,7 @@
 // render_loop.inl -- the path kernels' loop: runs until the launch's photons, or
 // the group's (GROUPS), are taken and the wave's lanes and stack are empty.
 // The text of a function body, included where FIELD, MODE, BATCH, JLDS, MM, GA,
-// SPLAT, GROUPS, STACK, SPLIT, the arguments S0 and A0, the shared arrays, group
+// SPLAT, STEPS, GROUPS, STACK, SPLIT, the arguments S0 and A0, the shared arrays, group
 // and wave_steps are declared.  As a function that takes the arguments by
 // reference, or by value, it made the 2^17-photon spline render 13 % slower
 // (136 -> 154 ms: the compiler keeps other scene scalars in registers).
@@ -108,6 +108,11 @@
             for (int k = 0; k < A0.spc; ++k) {
                 wave_steps += __popcll(__ballot(m));  // one ER step per marching lane
                 if (m) m = !march_step_jvp<FIELD>(h, tan, sl, S0, F, Lcut, A0.theta_dot);
+            }
+        } else if constexpr (STEPS) {
+            for (int k = 0; k < A0.spc; ++k) {
+                wave_steps += __popcll(__ballot(m));
+                if (m) m = !march_step<FIELD, false, MM, false, GA>(h, sl, S0, F, Lcut);
             }
         } else {
             march_chunk<FIELD, false, MM, GA, FIELD == kSpline>(h, sl, m, A0.spc, S0, F, Lcut, &scell, wave_steps);

@@ -80,3 +80,17 @@ def test_few_rays_match_the_oracle(gpu_ctx, axis, mode):
     assert np.abs(p[k] - po[k]).max() < 5e-8
     assert np.abs(dr[k] - do[k]).max() < 1e-5
     assert (np.abs(L[k] - Lo[k]) / Lo[k]).max() < 1e-5
+
+
+@pytest.mark.parametrize("mode", [0, 2, 5])
+@pytest.mark.parametrize("half_gap", [0.0005, 0.0019, 0.0021, 0.01])
+def test_many_rays_with_a_narrow_gap_are_the_few_ones(gpu_ctx, half_gap, mode):
+    """Rays that fill the launch's lanes take another loop where the gap planes
+    leave less than 0.4 of the block (4 of 10 mm) between them."""
+    d, tex, _ = scenes.transparent_cube(mode=mode, step=1e-4)
+    d.set(sgap_begin_loc_x=-half_gap, egap_end_loc_x=half_gap, n_max=2e-3, n_clip=2e-3)
+    sc = engine.Scene(gpu_ctx, d, tex)
+    many = sc.trace_rays((1 << 18) + 7, seed=3)
+    for a, b in zip(many, sc.trace_rays(5000, seed=3)):
+        assert torch.equal(a[:5000], b)
+    sc.close()
